@@ -65,7 +65,12 @@ struct CgState {
     int32_t extrap;         // extrapolation allowed (solver setting)
     // BiCGStab: rho = (r^, r), omega, and the pieces of omega
     double rho, omega, ts, tt;
+    // fast direct solver: applications when the problem stopped; its iterate
+    // is still the zero it started from
+    int32_t fast_iter, fast_zero;
 };
+
+struct FastSolver; // eq_fast.hip
 
 // One group of the batch's problems as the CG launches see it: global
 // problems [p0, p1); level-0 problem records [pi0, pi0 + npi) (the finish
@@ -286,6 +291,7 @@ struct eq_batch {
     eqk::InvJob* d_inv_jobs = nullptr;
     double* inv_scratch = nullptr;
     eqk::LevelProb** d_level_tables = nullptr;
+    eqk::FastSolver* fast = nullptr; // plans of the fast direct solver (NULL: the batch's grids or walls rule it out)
 };
 
 namespace eqk {
@@ -306,6 +312,14 @@ int refresh_cell_tensors(eq_batch* b);
 int set_trap_tensor(eq_batch* b, int trap, double Dx, double Dy, int on);
 // the coupling's tables and the fixed scratch's device address (at batch creation)
 int init_coupling(eq_batch* b);
+// the fast direct solver (eq_fast.hip): plans at batch creation; whether the
+// next step takes it; one solve (handled = false: the multigrid solver has to
+// go on); graphs and plans dropped
+int fast_build(eq_batch* b);
+bool fast_applies(const eq_batch* b);
+int fast_solve(eq_batch* b, bool profiling, bool* handled);
+void fast_drop_graphs(eq_batch* b);
+void fast_free(eq_batch* b);
 } // namespace eqk
 
 namespace eqk {

@@ -3724,6 +3724,7 @@ static void drop_graphs(eq_batch* b)
                         if (g) hipGraphExecDestroy(g);
                         g = nullptr;
                     }
+    fast_drop_graphs(b);
     for (hipGraphExec_t* g : {&b->g_init, &b->g_bicg, &b->g_ir2}) {
         if (*g) hipGraphExecDestroy(*g);
         *g = nullptr;
@@ -3812,6 +3813,34 @@ static int read_states(eq_batch* b)
 {
     EQ_HIP(hipMemcpyAsync(b->h_state, b->d_state, sizeof(CgState) * b->nprob, hipMemcpyDeviceToHost, b->stream));
     EQ_HIP(hipStreamSynchronize(b->stream));
+    return EQ_OK;
+}
+
+// Iterations, residuals and the verdict of a CG solve whose states are in h_state.
+static int report_solve(eq_batch* b, eq_step_stats* stats, std::chrono::steady_clock::time_point t0)
+{
+    int32_t itmax = 0, nconv = 0;
+    double relmax = 0.0;
+    for (int p = 0; p < b->nprob; ++p) {
+        const CgState& c = b->h_state[p];
+        const double rel = c.bb > 0 ? std::sqrt(c.rr_true / c.bb) : std::sqrt(c.rr_true);
+        b->iters[p] = c.iter;
+        b->relres[p] = rel;
+        itmax = std::max(itmax, c.iter);
+        relmax = std::max(relmax, rel);
+        if (c.rr_true <= c.tol2 * c.bb) ++nconv;
+    }
+    if (stats) {
+        stats->iterations_max = itmax;
+        stats->nconverged = nconv;
+        stats->relres_max = relmax;
+        stats->seconds = std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
+    }
+    if (nconv < b->nprob) {
+        char msg[128];
+        std::snprintf(msg, sizeof(msg), "max_iter reached above rtol (relres %.3e)", relmax);
+        return set_error(EQ_ERR_NOT_CONVERGED, msg);
+    }
     return EQ_OK;
 }
 
@@ -4072,30 +4101,9 @@ static int solve_all(eq_batch* b, eq_step_stats* stats)
                      b->stream, L0.all(), (const double*)b->u, b->xprev, b->xprev2, b->d_state);
     EQ_HIP(hipGetLastError());
     prof_collect(b);
-    int32_t itmax = 0, nconv = 0;
-    double relmax = 0.0;
-    for (int p = 0; p < b->nprob; ++p) {
-        const CgState& c = b->h_state[p];
-        const double rel = c.bb > 0 ? std::sqrt(c.rr_true / c.bb) : std::sqrt(c.rr_true);
-        b->iters[p] = c.iter;
-        b->relres[p] = rel;
-        itmax = std::max(itmax, c.iter);
-        relmax = std::max(relmax, rel);
-        if (c.rr_true <= c.tol2 * c.bb) ++nconv;
-    }
-    b->last_iters = itmax;
-    if (stats) {
-        stats->iterations_max = itmax;
-        stats->nconverged = nconv;
-        stats->relres_max = relmax;
-        stats->seconds = std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
-    }
-    if (nconv < b->nprob) {
-        char msg[128];
-        std::snprintf(msg, sizeof(msg), "max_iter reached above rtol (relres %.3e)", relmax);
-        return set_error(EQ_ERR_NOT_CONVERGED, msg);
-    }
-    return EQ_OK;
+    const int rc_solve = report_solve(b, stats, t0);
+    b->last_iters = *std::max_element(b->iters.begin(), b->iters.end());
+    return rc_solve;
 }
 
 } // namespace eqk
@@ -4416,7 +4424,47 @@ static int solve_ir(eq_batch* b, eq_step_stats* stats)
 }
 
 // precision of the multigrid x whether any problem carries a tensor field
+static int run_multigrid(eq_batch* b, eq_step_stats* stats);
+
+// The fast direct solver where it applies.  Where it gives up (a residual
+// that does not reach the tolerance), the multigrid solver takes the step over
+// from the same fields; the problems already solved keep their result.
 static int run_solve(eq_batch* b, eq_step_stats* stats)
+{
+    if (!fast_applies(b)) return run_multigrid(b, stats);
+    const auto t0 = std::chrono::steady_clock::now();
+    bool profiling = false, handled = true;
+    for (int k = 0; k < EQ_KERNEL_COUNT_; ++k) profiling = profiling || b->prof[k].enabled;
+    int rc = fast_solve(b, profiling, &handled);
+    if (rc != EQ_OK) return rc;
+    prof_collect(b);
+    if (handled) return report_solve(b, stats, t0);
+    const std::vector<CgState> solved(b->h_state, b->h_state + b->nprob);
+    const size_t bytes = sizeof(double) * b->levels[0].pool;
+    double* kept = nullptr;
+    if (hipMalloc((void**)&kept, bytes) != hipSuccess) return set_error(EQ_ERR_NOMEM, "solved fields");
+    hipStream_t s = b->stream;
+    rc = hipMemcpyAsync(kept, b->u, bytes, hipMemcpyDeviceToDevice, s) == hipSuccess
+             ? EQ_OK
+             : set_error(EQ_ERR_HIP, "solved fields");
+    const int mg = rc == EQ_OK ? run_multigrid(b, stats) : rc;
+    for (int p = 0; rc == EQ_OK && p < b->nprob; ++p) {
+        if (!solved[p].done) continue;
+        const LevelProb& P = b->levels[0].probs[p];
+        const size_t n = sizeof(double) * (size_t)P.pitch * (P.ny + 1);
+        for (double* v : {b->u, b->xprev})
+            if (hipMemcpyAsync(v + P.origin, kept + P.origin, n, hipMemcpyDeviceToDevice, s) != hipSuccess)
+                rc = set_error(EQ_ERR_HIP, "solved fields");
+        b->h_state[p] = solved[p];
+    }
+    if (hipStreamSynchronize(s) != hipSuccess && rc == EQ_OK) rc = set_error(EQ_ERR_HIP, "solved fields");
+    hipFree(kept);
+    if (rc != EQ_OK) return rc;
+    if (mg != EQ_OK && mg != EQ_ERR_NOT_CONVERGED) return mg;
+    return report_solve(b, stats, t0);
+}
+
+static int run_multigrid(eq_batch* b, eq_step_stats* stats)
 {
     const bool bicg = b->solver.kind == EQ_SOLVER_GMG_BICGSTAB || b->solver.kind == EQ_SOLVER_MIXED_GMG_BICGSTAB;
     if (!bicg)
@@ -4612,6 +4660,7 @@ int eq_batch_create(const eq_field_desc* descs, int32_t nprob, int32_t nspecies,
         }
     }
     if (rc == EQ_OK) rc = init_coupling(b);
+    if (rc == EQ_OK) rc = fast_build(b);
     if (rc != EQ_OK) {
         std::string keep = g_last_error;
         eq_batch_destroy(b);
@@ -4680,6 +4729,7 @@ void eq_batch_destroy(eq_batch* b)
     hipFree(b->d_inv_jobs);
     hipFree(b->inv_scratch);
     free_channels(b);
+    fast_free(b);
     hipFree(b->d_cell_traps);
     hipFree(b->d_cell_off);
     if (b->h_cell_off) hipHostFree(b->h_cell_off);

@@ -30,10 +30,12 @@ KERNEL_SMOOTH_COARSE, KERNEL_TRANSFER0, KERNEL_TRANSFER_COARSE, KERNEL_BOTTOM = 
 KERNEL_FINISH, KERNEL_SOLVE_ONCE, KERNEL_BICG_VEC, KERNEL_COUPLE_SETUP, KERNEL_BOUNDARY = 8, 9, 10, 11, 12
 KERNEL_COUNT = 13
 KERNEL_FAMILIES = {
-    KERNEL_STENCIL64: "Krylov operator apply (k_ap_dir, k_bicg_apply)",
+    KERNEL_STENCIL64: "Krylov operator apply (k_ap_dir, k_bicg_apply); fast solver: residual and forward transform "
+                      "(k_fast_forward)",
     KERNEL_SMOOTH: "finest-level way up: correction and sweeps (k_level_up; k_smooth, k_presmooth2, "
                    "k_prolong_smooth on level 0)",
-    KERNEL_CG_UPDATE: "Krylov x, r update + dots (k_update, k_bicg_x)",
+    KERNEL_CG_UPDATE: "Krylov x, r update + dots (k_update, k_bicg_x); fast solver: backward transform and update "
+                      "(k_fast_backward)",
     KERNEL_COUPLE: "cell sample/deposit per tile (k_tile_couple)",
     KERNEL_SMOOTH_COARSE: "coarse-level way up: correction and sweeps (k_level_up; k_smooth, k_presmooth2, "
                           "k_prolong_smooth)",
@@ -41,9 +43,10 @@ KERNEL_FAMILIES = {
                       "k_residual_restrict, k_prolong on level 0)",
     KERNEL_TRANSFER_COARSE: "coarse-level way down: sweeps, residual, restriction (k_level_down; k_residual, "
                             "k_restrict, k_residual_restrict)",
-    KERNEL_BOTTOM: "LDS bottom V-cycle (k_bottom, k_cast_in, k_cast_out)",
+    KERNEL_BOTTOM: "LDS bottom V-cycle (k_bottom, k_cast_in, k_cast_out); fast solver: line solves (k_fast_lines)",
     KERNEL_FINISH: "per-problem reduction finish (k_finish)",
-    KERNEL_SOLVE_ONCE: "once per solve (k_rhs, k_init, k_true_residual, k_keep, first sweep, k_copy)",
+    KERNEL_SOLVE_ONCE: "once per solve (k_rhs, k_init, k_true_residual, k_keep, first sweep, k_copy, "
+                       "k_fast_check, k_fast_commit)",
     KERNEL_BICG_VEC: "BiCGStab vector updates (k_bicg_p, k_bicg_s)",
     KERNEL_COUPLE_SETUP: "cell geometry, pair scan and sort, tile bounds, per-cell sums",
     KERNEL_BOUNDARY: "channels, boundary wells and values, flux",
