@@ -16,9 +16,14 @@
 // The finite-difference scheme is separable exactly.
 //
 // Measured per time step, couple + solve + fields out, against the V-cycle
-// CG: 2000x1000, 2 species 2.57 -> 0.48 ms (FP64 3.03 -> 0.60), 1237x611 (a
-// chirp length) 1.95 -> 0.43, 12 uneven traps 3.32 -> 1.34, 512 uneven traps
-// 69.5 -> 43.6; errors against a 64-bit solve 4e-15 to 6e-13.
+// CG: 2000x1000, 2 species 2.58 -> 0.40 ms (FP64 3.04 -> 0.46), 1237x611 (a
+// chirp length) 2.02 -> 0.34, 12 uneven traps 3.32 -> 1.02, 512 uneven traps
+// 69.4 -> 28.0; errors against a 64-bit solve 4e-15 to 6e-13.
+//
+// What bounds the transforms: vector issue and latency, not bandwidth
+// (2000x1000: forward 34 us, backward 28, where the bytes take 18 and 14).
+// They are compiled for 64 registers, eight waves a SIMD: at 82 to 119
+// registers the same launch took two rounds of blocks and 59 and 34 us.
 //
 // P^-1: trigonometric transform along x (the eigenvectors of the x matrices:
 // cosines for closed walls, sines for held ones, quarter-wave cosines for one
@@ -66,7 +71,9 @@ enum FastEnds { kEndsNN = 0, kEndsDD = 1, kEndsND = 2, kEndsDN = 3 };
 struct FastPlan {
     int32_t N, n, M, chirp;
     int32_t nstages;
-    int32_t radix[kFastMaxStages];
+    struct Pass {
+        int32_t R, m, Ns, step; // radix, M / R, product of the radices before, m / Ns
+    } pass[kFastMaxStages];
     int64_t tw;     // M: exp(-2 pi i k / M)
     int64_t quart;  // N + 1: exp(-pi i j / (2 N))
     int64_t ch;     // chirp: n values exp(-pi i j^2 / n)
@@ -76,6 +83,16 @@ struct FastPlan {
 struct FastProb {
     int32_t plan, ends;
     int32_t pair0, npairs;  // this problem's slots of row-pair partials
+};
+
+// The rows of a problem's operator and right-hand side by place: bottom row,
+// between, top row by left column, between, right column.  A node at a wall
+// then costs the same loads as any other (the frame around a field is zero),
+// only other coefficients; evaluating the element counts there made the few
+// blocks of wall rows the last to finish, at twice the launch's time.
+struct FastRows {
+    Row<double> a[3][3];
+    double b[3][3][8]; // c, w, e, s, n, sw, ne of M, and the sources
 };
 
 // a block's work: problem and row pair (forward, backward) or mode group
@@ -95,6 +112,7 @@ struct FastSolver {
     int32_t nline = 0, line_c = 0, line_rows = 0;
     FastPlan* d_plans = nullptr;
     FastProb* d_probs = nullptr;
+    FastRows* d_rows = nullptr;
     FastJob* d_jobs = nullptr;   // row pairs, class by class
     FastJob* d_lines = nullptr;  // mode groups
     void* d_tables = nullptr;
@@ -188,6 +206,47 @@ __device__ __forceinline__ void dft(Cx<T> (&v)[R])
         v[4] = {m1.x - n1.y, m1.y + n1.x};
         v[2] = {m2.x + n2.y, m2.y - n2.x};
         v[3] = {m2.x - n2.y, m2.y + n2.x};
+    } else if constexpr (R == 6 || R == 10) {
+        // 2 x R/2 with coprime factors (Good-Thomas): no twiddles
+        constexpr int H = R / 2;
+        Cx<T> e[H], o[H];
+#pragma unroll
+        for (int q = 0; q < H; ++q) {
+            const Cx<T> a = v[(2 * q) % R], b = v[(2 * q + H) % R];
+            e[q] = a + b;
+            o[q] = a - b;
+        }
+        dft<T, H>(e);
+        dft<T, H>(o);
+        // output k: residues (k mod 2, k mod H)
+#pragma unroll
+        for (int k = 0; k < R; ++k) v[k] = (k & 1) ? o[k % H] : e[k % H];
+    } else if constexpr (R == 9) {
+        const T c1 = (T)0.76604444311897803520, s1 = (T)0.64278760968653932632;
+        const T c2 = (T)0.17364817766693034885, s2 = (T)0.98480775301220805937;
+        const T c4 = (T)-0.93969262078590838405, s4 = (T)0.34202014332566873304;
+        Cx<T> a[3], b[3], c[3];
+#pragma unroll
+        for (int q = 0; q < 3; ++q) {
+            a[q] = v[3 * q];
+            b[q] = v[3 * q + 1];
+            c[q] = v[3 * q + 2];
+        }
+        dft<T, 3>(a);
+        dft<T, 3>(b);
+        dft<T, 3>(c);
+        b[1] = mul(b[1], Cx<T>{c1, -s1});
+        b[2] = mul(b[2], Cx<T>{c2, -s2});
+        c[1] = mul(c[1], Cx<T>{c2, -s2});
+        c[2] = mul(c[2], Cx<T>{c4, -s4});
+#pragma unroll
+        for (int q = 0; q < 3; ++q) {
+            Cx<T> t[3] = {a[q], b[q], c[q]};
+            dft<T, 3>(t);
+            v[q] = t[0];
+            v[q + 3] = t[1];
+            v[q + 6] = t[2];
+        }
     } else {
         static_assert(R == 7, "radix");
         const T c1 = (T)0.62348980185873353053, c2 = (T)-0.22252093395631440429, c3 = (T)-0.90096886790241912624;
@@ -212,26 +271,25 @@ __device__ __forceinline__ void dft(Cx<T> (&v)[R])
 
 // ------------------------------------------------------------ transforms in LDS
 
-// one element of padding per 16: a wave's strided writes of the early passes
-// then spread over the banks
-__host__ __device__ __forceinline__ int pad16(int i) { return i + (i >> 4); }
-
 // One Stockham pass of radix R in place: every value is held in registers
-// across the barrier between its read and its write.  M <= V NT.
-template <typename T, int R, int NT, int V>
-__device__ __forceinline__ void fft_pass(Cx<T>* s, int M, int Ns, const Cx<T>* __restrict__ tw)
+// across the barrier between its read and its write.  M <= V NT.  Output
+// element i goes to store(i, value).  The passes run odd and singly even
+// radices first (see make_plan), so the strided writes of the early ones
+// spread over the LDS banks without padding.
+template <typename T, int R, int NT, int V, typename S>
+__device__ __forceinline__ void fft_pass(Cx<T>* s, const FastPlan::Pass& ps, const Cx<T>* __restrict__ tw, S&& store)
 {
     constexpr int B = (V + R - 1) / R;
-    const int m = M / R;
+    const int m = ps.m, Ns = ps.Ns;
     const float inv = 1.0f / (float)Ns;
-    const int step = m / Ns;
+    const uint32_t step = (uint32_t)ps.step * (uint32_t)sizeof(Cx<T>);
     Cx<T> v[B][R];
 #pragma unroll
     for (int b = 0; b < B; ++b) {
         const int k = (int)threadIdx.x + b * NT;
         if (k < m)
 #pragma unroll
-            for (int r = 0; r < R; ++r) v[b][r] = s[pad16(k + r * m)];
+            for (int r = 0; r < R; ++r) v[b][r] = s[k + r * m];
     }
     __syncthreads();
 #pragma unroll
@@ -241,83 +299,92 @@ __device__ __forceinline__ void fft_pass(Cx<T>* s, int M, int Ns, const Cx<T>* _
             // k = p Ns + q with q the position inside the finished sub-transforms
             const int p = (int)(((float)k + 0.5f) * inv), q = k - p * Ns;
             if (Ns > 1) {
-                const int t = q * step;
+                const uint32_t t = (uint32_t)q * step;
 #pragma unroll
-                for (int r = 1; r < R; ++r)
-                    v[b][r] = mul(v[b][r], *(const Cx<T>*)((const char*)tw + (uint32_t)(t * r) * (uint32_t)sizeof(Cx<T>)));
+                for (int r = 1; r < R; ++r) v[b][r] = mul(v[b][r], *(const Cx<T>*)((const char*)tw + t * (uint32_t)r));
             }
             dft<T, R>(v[b]);
             const int o = p * Ns * R + q;
 #pragma unroll
-            for (int r = 0; r < R; ++r) s[pad16(o + r * Ns)] = v[b][r];
+            for (int r = 0; r < R; ++r) store(o + r * Ns, v[b][r]);
         }
     }
-    __syncthreads();
 }
 
-template <typename T, int NT, int V>
-__device__ __forceinline__ void fft_lds(Cx<T>* s, const FastPlan& pl, const Cx<T>* __restrict__ tab)
+// The pass's sizes come from its record: worked out in place, every radix's
+// would be kept in registers through the loop over the passes.
+template <typename T, int NT, int V, typename S>
+__device__ __forceinline__ void fft_radix(Cx<T>* s, const FastPlan::Pass& ps, const Cx<T>* __restrict__ tw, S&& store)
+{
+    switch (ps.R) {
+    case 10: fft_pass<T, 10, NT, V>(s, ps, tw, store); break;
+    case 9: fft_pass<T, 9, NT, V>(s, ps, tw, store); break;
+    case 8: fft_pass<T, 8, NT, V>(s, ps, tw, store); break;
+    case 7: fft_pass<T, 7, NT, V>(s, ps, tw, store); break;
+    case 6: fft_pass<T, 6, NT, V>(s, ps, tw, store); break;
+    case 5: fft_pass<T, 5, NT, V>(s, ps, tw, store); break;
+    case 4: fft_pass<T, 4, NT, V>(s, ps, tw, store); break;
+    case 3: fft_pass<T, 3, NT, V>(s, ps, tw, store); break;
+    default: fft_pass<T, 2, NT, V>(s, ps, tw, store); break;
+    }
+}
+
+// The M-point transform of the row in LDS; the last pass hands its outputs to
+// `last` (after a barrier behind the pass's reads, so it may write the row).
+template <typename T, int NT, int V, typename S>
+__device__ __forceinline__ void fft_lds(Cx<T>* s, const FastPlan& pl, const Cx<T>* __restrict__ tab, S&& last)
 {
     const Cx<T>* tw = tab + pl.tw;
-    int Ns = 1;
-    for (int k = 0; k < pl.nstages; ++k) {
-        const int R = pl.radix[k];
-        switch (R) {
-        case 8: fft_pass<T, 8, NT, V>(s, pl.M, Ns, tw); break;
-        case 7: fft_pass<T, 7, NT, V>(s, pl.M, Ns, tw); break;
-        case 5: fft_pass<T, 5, NT, V>(s, pl.M, Ns, tw); break;
-        case 4: fft_pass<T, 4, NT, V>(s, pl.M, Ns, tw); break;
-        case 3: fft_pass<T, 3, NT, V>(s, pl.M, Ns, tw); break;
-        default: fft_pass<T, 2, NT, V>(s, pl.M, Ns, tw); break;
-        }
-        Ns *= R;
+    const int n = pl.nstages - 1;
+    for (int k = 0; k < n; ++k) {
+        fft_radix<T, NT, V>(s, pl.pass[k], tw, [&](int i, Cx<T> v) { s[i] = v; });
+        __syncthreads();
     }
+    fft_radix<T, NT, V>(s, pl.pass[n], tw, last);
 }
 
-// The plan's n-point transform of the row placed with put_at: the smooth
-// length directly, or the chirp convolution (the second transform runs on the
-// conjugate, so its result is conjugate).
-template <typename T, int NT, int V>
-__device__ __forceinline__ void row_transform(Cx<T>* s, const FastPlan& pl, const Cx<T>* __restrict__ tab)
+// The plan's n-point transform of the row placed with put_at, elements 0 .. N
+// to out(k, value): the smooth length directly, or the chirp convolution (its
+// second transform runs on the conjugate, so its result is conjugate).
+template <typename T, int NT, int V, typename S>
+__device__ __forceinline__ void row_transform(Cx<T>* s, const FastPlan& pl, const Cx<T>* __restrict__ tab, S&& out)
 {
+    const int N = pl.N;
     __syncthreads();
     if (!pl.chirp) {
-        fft_lds<T, NT, V>(s, pl, tab);
+        fft_lds<T, NT, V>(s, pl, tab, [&](int k, Cx<T> v) {
+            if (k <= N) out(k, v);
+        });
         return;
     }
     const Cx<T>* h = tab + pl.hh;
-    for (int pass = 0; pass < 2; ++pass) {
-        fft_lds<T, NT, V>(s, pl, tab);
-        if (pass == 0) {
-            for (int k = threadIdx.x; k < pl.M; k += NT) {
-                const Cx<T> p = mul(s[pad16(k)], h[k]);
-                s[pad16(k)] = {p.x, -p.y};
-            }
-            __syncthreads();
-        }
-    }
+    fft_lds<T, NT, V>(s, pl, tab, [&](int k, Cx<T> v) {
+        const Cx<T> p = mul(v, h[k]);
+        s[k] = {p.x, -p.y};
+    });
+    __syncthreads();
+    const Cx<T>* ch = tab + pl.ch;
+    fft_lds<T, NT, V>(s, pl, tab, [&](int k, Cx<T> v) {
+        if (k <= N) out(k, mul(Cx<T>{v.x, -v.y}, ch[k]));
+    });
 }
 // element j of the period-n row, -n/2 <= j <= n/2
 template <typename T>
 __device__ __forceinline__ void put_at(Cx<T>* s, const FastPlan& pl, const Cx<T>* __restrict__ tab, int j, Cx<T> v)
 {
     if (pl.chirp) v = mul(v, tab[pl.ch + (j < 0 ? -j : j)]);
-    s[pad16(j < 0 ? j + pl.M : j)] = v;
-}
-template <typename T>
-__device__ __forceinline__ Cx<T> get_at(const Cx<T>* s, const FastPlan& pl, const Cx<T>* __restrict__ tab, int k)
-{
-    const Cx<T> v = s[pad16(k)];
-    if (!pl.chirp) return v;
-    return mul(Cx<T>{v.x, -v.y}, tab[pl.ch + k]);
+    s[j < 0 ? j + pl.M : j] = v;
 }
 // the chirp's gap between the placed rows: elements a .. b are zero
 template <typename T, int NT>
 __device__ __forceinline__ void clear_gap(Cx<T>* s, const FastPlan& pl, int a, int b)
 {
     if (!pl.chirp) return;
-    for (int k = a + (int)threadIdx.x; k <= b; k += NT) s[pad16(k)] = {(T)0, (T)0};
+    for (int k = a + (int)threadIdx.x; k <= b; k += NT) s[k] = {(T)0, (T)0};
 }
+
+// waves per SIMD the transform kernels are compiled for
+constexpr int fast_waves(size_t elem, int NT, int V) { return V > kFastValues ? 4 : elem == 4 ? 8 : 4; }
 
 // ------------------------------------------------------------ residual rows
 
@@ -337,82 +404,97 @@ __device__ __forceinline__ double wave_add(double v)
     return v;
 }
 
-// r = b - A x at node (i, j) near a wall, b = M u + sources; held neighbours
-// take their wall value.  zero_x: the iterate is zero on the free nodes.
-__device__ __forceinline__ double residual_wall(const LevelProb& P, int i, int j, const double* __restrict__ u,
-                                                const double* __restrict__ x, bool zero_x, double& bv)
-{
-    const int64_t k = P.origin + (int64_t)i * P.pitch + j;
-    const int pt = P.pitch;
-    bv = rhs_row(P, i, j, u[k], u[k - 1], u[k + 1], u[k - pt], u[k + pt], u[k - pt - 1], u[k + pt + 1]);
-    auto val = [&](int ii, int jj, int64_t kk) -> double {
-        if (is_dirichlet_nb(P, ii, jj)) return dirichlet_value(P, ii, jj);
-        return zero_x ? 0.0 : x[kk];
-    };
-    const Row<double> rc = row_coefs_at<double>(P, i, j);
-    return bv - row_apply<false>(rc, val(i, j, k), val(i, j - 1, k - 1), val(i, j + 1, k + 1), val(i - 1, j, k - pt),
-                                 val(i + 1, j, k + pt), val(i - 1, j - 1, k - pt - 1), val(i + 1, j + 1, k + pt + 1));
-}
+struct PairWindow { // rows i0-1 .. i0+2 of column j, and of its neighbours as far as the two rows need them
+    double m[4], w[3], e[3];
+    __device__ __forceinline__ void load(const double* __restrict__ v, int j, const int (&row)[4])
+    {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) m[q] = v[row[q] + j];
+#pragma unroll
+        for (int q = 0; q < 3; ++q) {
+            w[q] = v[row[q] + j - 1];
+            e[q] = v[row[q + 1] + j + 1];
+        }
+    }
+    // any row's coefficients
+    __device__ __forceinline__ double apply(const Row<double>& r, int k) const
+    {
+        return row_apply<false>(r, m[k + 1], w[k + 1], e[k], m[k], m[k + 2], w[k], e[k + 1]);
+    }
+    __device__ __forceinline__ double rhs(const double* c, int k) const
+    {
+        return c[0] * m[k + 1] + ((c[1] * w[k + 1] + c[2] * e[k]) + (c[3] * m[k] + c[4] * m[k + 2])) +
+               (c[5] * w[k] + c[6] * e[k + 1]) + c[7];
+    }
+    // a row off the walls: its neighbours' weights are equal, or equal by axis
+    __device__ __forceinline__ double apply_inner(double mc, double mo, double kx, double ky, int k) const
+    {
+        const double c = m[k + 1];
+        return (kx * ((c - w[k + 1]) + (c - e[k])) + ky * ((c - m[k]) + (c - m[k + 2]))) + rhs_inner(mc, mo, k);
+    }
+    __device__ __forceinline__ double rhs_inner(double mc, double mo, int k) const
+    {
+        return mc * m[k + 1] + mo * (((w[k + 1] + e[k]) + (m[k] + m[k + 2])) + (w[k] + e[k + 1]));
+    }
+};
 
-// Rows i0 and i0 + 1 of the residual, column by column; f(j, r0, r1) takes
-// them.  Sums r^2 and (row-replaced) b^2 into acc.
+// Rows i0 and i0 + 1 of the residual b - A x, b = M u + sources, column by
+// column; f(j, r0, r1) takes them (0 on held nodes, where x holds the wall
+// value).  Sums r^2, and with want_b the row-replaced b^2, into acc.
 template <int NT, typename F>
-__device__ __forceinline__ void residual_pair(const LevelProb& P, int i0, const double* __restrict__ u,
-                                              const double* __restrict__ x, bool zero_x, double (&acc)[2], F&& f)
+__device__ __forceinline__ void residual_pair(const LevelProb& P, const FastRows& tab, int i0,
+                                              const double* __restrict__ u, const double* __restrict__ x, bool want_b,
+                                              double (&acc)[2], F&& f)
 {
     const int nx = P.nx, ny = P.ny, pt = P.pitch;
-    // the two rows and their neighbours lie off every wall row
-    const bool rows = i0 > 1 && i0 + 2 < ny;
-    const Row<double> rc = P.rin;
-    const double c0 = P.fd ? P.mh0 : 6.0 * P.mh0, c1 = P.fd ? 0.0 : 2.0 * P.mo0, cs = P.fd ? P.fsrcf : 6.0 * P.src;
+    const bool in1 = i0 + 1 <= ny;
     const double* __restrict__ ur = u + P.origin + (int64_t)i0 * pt;
     const double* __restrict__ xr = x + P.origin + (int64_t)i0 * pt;
+    const int row[4] = {-pt, 0, pt, in1 ? 2 * pt : pt}; // (the frame ends at row ny + 1)
+    const bool inner = i0 > 0 && i0 + 1 < ny;
+    // one column with the table's rows (column class cc)
+    auto by_table = [&](int j, int cc) {
+        const int c0 = i0 == 0 ? 0 : i0 == ny ? 2 : 1, c1 = i0 + 1 >= ny ? 2 : 1;
+        PairWindow U, X;
+        U.load(ur, j, row);
+        X.load(xr, j, row);
+        double b0 = U.rhs(tab.b[c0][cc], 0), b1 = in1 ? U.rhs(tab.b[c1][cc], 1) : 0.0;
+        double r0 = b0 - X.apply(tab.a[c0][cc], 0), r1 = in1 ? b1 - X.apply(tab.a[c1][cc], 1) : 0.0;
+        if (is_dirichlet(P, i0, j)) {
+            r0 = 0.0;
+            b0 = want_b ? dirichlet_value(P, i0, j) : 0.0;
+        }
+        if (in1 && is_dirichlet(P, i0 + 1, j)) {
+            r1 = 0.0;
+            b1 = want_b ? dirichlet_value(P, i0 + 1, j) : 0.0;
+        }
+        acc[0] += r0 * r0 + r1 * r1;
+        acc[1] += b0 * b0 + b1 * b1;
+        f(j, r0, r1);
+    };
+    // the wall columns: one lane of a wave each, first
+    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
 #pragma unroll 1
-    for (int j = threadIdx.x; j <= nx; j += NT) {
-        double r0 = 0.0, r1 = 0.0;
-        if (rows && j > 1 && j + 1 < nx) {
-            double um[4], uw[3], ue[3];
-#pragma unroll
-            for (int q = 0; q < 4; ++q) um[q] = ur[j + (q - 1) * pt];
-#pragma unroll
-            for (int q = 0; q < 3; ++q) {
-                uw[q] = ur[j - 1 + (q - 1) * pt];
-                ue[q] = ur[j + 1 + q * pt];
-            }
-            double xm[4] = {0, 0, 0, 0}, xw[3] = {0, 0, 0}, xe[3] = {0, 0, 0};
-            if (!zero_x) {
-#pragma unroll
-                for (int q = 0; q < 4; ++q) xm[q] = xr[j + (q - 1) * pt];
-#pragma unroll
-                for (int q = 0; q < 3; ++q) {
-                    xw[q] = xr[j - 1 + (q - 1) * pt];
-                    xe[q] = xr[j + 1 + q * pt];
-                }
-            }
-            const double b0 = c0 * um[1] + c1 * (((uw[1] + ue[0]) + (um[0] + um[2])) + (uw[0] + ue[1])) + cs;
-            const double b1 = c0 * um[2] + c1 * (((uw[2] + ue[1]) + (um[1] + um[3])) + (uw[1] + ue[2])) + cs;
-            r0 = b0 - row_apply<false>(rc, xm[1], xw[1], xe[0], xm[0], xm[2], xw[0], xe[1]);
-            r1 = b1 - row_apply<false>(rc, xm[2], xw[2], xe[1], xm[1], xm[3], xw[1], xe[2]);
+    for (int e = wave; e < 2; e += NT / 64)
+        if ((threadIdx.x & 63) == 0) by_table(e ? nx : 0, e ? 2 : 0);
+    if (inner) {
+        const Row<double>& ra = tab.a[1][1];
+        const double mc = ra.mc, mo = ra.mw, kx = ra.kw, ky = ra.ks;
+        const double c0 = tab.b[1][1][0], c1 = tab.b[1][1][1], cs = tab.b[1][1][7];
+#pragma unroll 1
+        for (int j = 1 + (int)threadIdx.x; j < nx; j += NT) {
+            PairWindow U, X;
+            U.load(ur, j, row);
+            X.load(xr, j, row);
+            const double b0 = U.rhs_inner(c0, c1, 0) + cs, b1 = U.rhs_inner(c0, c1, 1) + cs;
+            const double r0 = b0 - X.apply_inner(mc, mo, kx, ky, 0), r1 = b1 - X.apply_inner(mc, mo, kx, ky, 1);
             acc[0] += r0 * r0 + r1 * r1;
             acc[1] += b0 * b0 + b1 * b1;
-        } else {
-#pragma unroll
-            for (int w = 0; w < 2; ++w) {
-                const int i = i0 + w;
-                if (i > ny) continue;
-                if (is_dirichlet(P, i, j)) {
-                    const double g = dirichlet_value(P, i, j);
-                    acc[1] += g * g;
-                    continue;
-                }
-                double bv;
-                const double rv = residual_wall(P, i, j, u, x, zero_x, bv);
-                acc[0] += rv * rv;
-                acc[1] += bv * bv;
-                (w ? r1 : r0) = rv;
-            }
+            f(j, r0, r1);
         }
-        f(j, r0, r1);
+    } else {
+#pragma unroll 1
+        for (int j = 1 + (int)threadIdx.x; j < nx; j += NT) by_table(j, 1);
     }
 }
 
@@ -441,13 +523,13 @@ __device__ __forceinline__ void block_pair(double (&v)[2])
 
 // Residual of the iterate and its transform along x, two rows a block.
 // k: applications done so far in this solve (0: the first residual, which
-// also takes ||b||^2; the iterate is the last solution, or zero where none is
-// kept).  start: this launch begins a chunk of the host's loop.
+// also takes ||b||^2).  start: this launch begins a chunk of the host's loop.
 template <typename T, int NT, int V>
-__global__ __launch_bounds__(NT, (sizeof(T) == 4 || NT == 1024) ? 4 : 2) void k_fast_forward(const FastJob* __restrict__ jobs, int njobs,
+__global__ __launch_bounds__(NT, fast_waves(sizeof(T), NT, V)) void k_fast_forward(const FastJob* __restrict__ jobs, int njobs,
                                                      const LevelProb* __restrict__ probs,
-                                                     const FastProb* __restrict__ fp, const FastPlan* __restrict__ plans,
-                                                     const Cx<T>* __restrict__ tab, const double* __restrict__ u,
+                                                     const FastProb* __restrict__ fp, const FastRows* __restrict__ rows,
+                                                     const FastPlan* __restrict__ plans, const Cx<T>* __restrict__ tab,
+                                                     const double* __restrict__ u,
                                                      const double* __restrict__ x, T* __restrict__ out,
                                                      double* __restrict__ partial, CgState* st, int k, int start)
 {
@@ -466,12 +548,11 @@ __global__ __launch_bounds__(NT, (sizeof(T) == 4 || NT == 1024) ? 4 : 2) void k_
     const FastProb f = fp[job.prob];
     const FastPlan& pl = plans[f.plan];
     const int N = pl.N, i0 = 2 * job.at;
-    const bool zero_x = k == 0 && cs.have_prev == 0;
     double acc[2] = {0.0, 0.0};
     const int ends = f.ends;
     const T two = (T)2;
     clear_gap<T, NT>(s, pl, N + 1, pl.M - N);
-    residual_pair<NT>(P, i0, u, x, zero_x, acc, [&](int j, double r0, double r1) {
+    residual_pair<NT>(P, rows[job.prob], i0, u, x, k == 0, acc, [&](int j, double r0, double r1) {
         Cx<T> v = {(T)r0, (T)r1};
         if (ends == kEndsNN) {
             if (j == 0 || j == N) {
@@ -500,22 +581,22 @@ __global__ __launch_bounds__(NT, (sizeof(T) == 4 || NT == 1024) ? 4 : 2) void k_
         partial[2 * (int64_t)(f.pair0 + job.at)] = acc[0];
         partial[2 * (int64_t)(f.pair0 + job.at) + 1] = acc[1];
     }
-    row_transform<T, NT, V>(s, pl, tab);
     T* __restrict__ o0 = out + P.origin + (int64_t)i0 * P.pitch;
     const bool second = i0 + 1 <= P.ny;
-    for (int q = threadIdx.x; q <= N; q += NT) {
-        const Cx<T> v = get_at(s, pl, tab, q);
+    const int pitch = P.pitch;
+    row_transform<T, NT, V>(s, pl, tab, [&](int q, Cx<T> v) {
         const Cx<T> w = ends == kEndsDD ? Cx<T>{-v.y, v.x} : v;
         o0[q] = w.x;
-        if (second) o0[q + P.pitch] = w.y;
-    }
+        if (second) o0[q + pitch] = w.y;
+    });
 }
 
 // The residual alone: the confirmation after a chunk of applications.
 __global__ __launch_bounds__(256) void k_fast_check(const FastJob* __restrict__ jobs, int njobs,
                                                     const LevelProb* __restrict__ probs,
-                                                    const FastProb* __restrict__ fp, const double* __restrict__ u,
-                                                    const double* __restrict__ x, double* __restrict__ partial,
+                                                    const FastProb* __restrict__ fp, const FastRows* __restrict__ rows,
+                                                    const double* __restrict__ u, const double* __restrict__ x,
+                                                    double* __restrict__ partial,
                                                     const CgState* __restrict__ st)
 {
     const int t = swizzled_block();
@@ -524,7 +605,7 @@ __global__ __launch_bounds__(256) void k_fast_check(const FastJob* __restrict__ 
     const LevelProb& P = probs[job.prob];
     if (st[P.prob].done) return;
     double acc[2] = {0.0, 0.0};
-    residual_pair<256>(P, 2 * job.at, u, x, false, acc, [](int, double, double) {});
+    residual_pair<256>(P, rows[job.prob], 2 * job.at, u, x, false, acc, [](int, double, double) {});
     block_pair<256>(acc);
     if (threadIdx.x == 0) partial[2 * (int64_t)(fp[job.prob].pair0 + job.at)] = acc[0];
 }
@@ -605,10 +686,7 @@ __global__ void k_fast_lines(const FastJob* __restrict__ jobs, int njobs, const 
     if (k > 0) bb = cs.bb;
     const bool conv = rr <= cs.tol2 * bb, stop = conv || k >= cs.max_iter;
     if (job.at == 0 && threadIdx.x == 0) {
-        if (k == 0) {
-            cs.bb = bb;
-            cs.fast_zero = stop && cs.have_prev == 0;
-        }
+        if (k == 0) cs.bb = bb;
         cs.done = stop ? 1 : 0;
         if (stop) {
             cs.fast_iter = k;
@@ -718,12 +796,12 @@ __global__ void k_fast_lines(const FastJob* __restrict__ jobs, int njobs, const 
 
 // Transform back along x and x += z, two rows a block.
 template <typename T, int NT, int V>
-__global__ __launch_bounds__(NT, (sizeof(T) == 4 || NT == 1024) ? 4 : 2) void k_fast_backward(const FastJob* __restrict__ jobs, int njobs,
+__global__ __launch_bounds__(NT, fast_waves(sizeof(T), NT, V)) void k_fast_backward(const FastJob* __restrict__ jobs, int njobs,
                                                       const LevelProb* __restrict__ probs,
                                                       const FastProb* __restrict__ fp,
                                                       const FastPlan* __restrict__ plans,
                                                       const Cx<T>* __restrict__ tab, const T* __restrict__ in,
-                                                      double* __restrict__ x, const CgState* __restrict__ st, int k)
+                                                      double* __restrict__ x, const CgState* __restrict__ st)
 {
     extern __shared__ char lds_raw[];
     Cx<T>* s = (Cx<T>*)lds_raw;
@@ -736,7 +814,6 @@ __global__ __launch_bounds__(NT, (sizeof(T) == 4 || NT == 1024) ? 4 : 2) void k_
     const FastProb f = fp[job.prob];
     const FastPlan& pl = plans[f.plan];
     const int N = pl.N, i0 = 2 * job.at, ends = f.ends;
-    const bool first = k == 0 && cs.have_prev == 0; // the iterate was zero
     const bool second = i0 + 1 <= P.ny;
     const T* __restrict__ r0 = in + P.origin + (int64_t)i0 * P.pitch;
     const T* __restrict__ r1 = second ? r0 + P.pitch : r0;
@@ -754,19 +831,21 @@ __global__ __launch_bounds__(NT, (sizeof(T) == 4 || NT == 1024) ? 4 : 2) void k_
             put_at(s, pl, tab, pl.chirp ? -q - 1 : 2 * N - 1 - q, v);
         }
     }
-    row_transform<T, NT, V>(s, pl, tab);
     double* __restrict__ xr = x + P.origin + (int64_t)i0 * P.pitch;
-    for (int j = threadIdx.x; j <= N; j += NT) {
-        const int jj = ends == kEndsDN ? N - j : j;
-        Cx<T> v = get_at(s, pl, tab, jj);
+    const int pitch = P.pitch;
+    const bool held0 = i0 == 0 && (P.dmask & (1 << kBottom)), held1 = i0 + 1 == P.ny && (P.dmask & (1 << kTop));
+    const bool top0 = i0 == P.ny && (P.dmask & (1 << kTop));
+    const int jlo = (P.dmask & (1 << kLeft)) ? 1 : 0, jhi = (P.dmask & (1 << kRight)) ? N - 1 : N;
+    row_transform<T, NT, V>(s, pl, tab, [&](int jj, Cx<T> v) {
+        const int j = ends == kEndsDN ? N - jj : jj;
         if (ends == kEndsDD)
             v = Cx<T>{-v.y, v.x};
         else if (ends >= kEndsND)
             v = mul(v, tab[pl.quart + jj]);
-        if (!is_dirichlet(P, i0, j)) xr[j] = first ? (double)v.x : xr[j] + (double)v.x;
-        if (second && !is_dirichlet(P, i0 + 1, j))
-            xr[j + P.pitch] = first ? (double)v.y : xr[j + P.pitch] + (double)v.y;
-    }
+        if (j < jlo || j > jhi) return;
+        if (!held0 && !top0) xr[j] += (double)v.x;
+        if (second && !held1) xr[j + pitch] += (double)v.y;
+    });
 }
 
 // The chunk's end: every block takes its problem's residual norm, and where
@@ -775,7 +854,7 @@ __global__ __launch_bounds__(NT, (sizeof(T) == 4 || NT == 1024) ? 4 : 2) void k_
 __global__ __launch_bounds__(256) void k_fast_commit(const FastJob* __restrict__ jobs, int njobs,
                                                      const LevelProb* __restrict__ probs,
                                                      const FastProb* __restrict__ fp, double* __restrict__ u,
-                                                     double* __restrict__ x, const double* __restrict__ partial,
+                                                     const double* __restrict__ x, const double* __restrict__ partial,
                                                      CgState* st, int k)
 {
     __shared__ double red[16];
@@ -792,7 +871,6 @@ __global__ __launch_bounds__(256) void k_fast_commit(const FastJob* __restrict__
     if (was == 2) return;
     // (a block that already reads the first block's `done` takes the same way)
     const bool conv = rr <= cs.tol2 * cs.bb, over = was || conv || k >= cs.max_iter;
-    const bool zero = cs.fast_zero != 0;
     if (job.at == 0 && threadIdx.x == 0) {
         if (!was) {
             cs.fast_iter = k;
@@ -810,14 +888,34 @@ __global__ __launch_bounds__(256) void k_fast_commit(const FastJob* __restrict__
         const int i = 2 * job.at + w;
         if (i > P.ny) break;
         const int64_t r = P.origin + (int64_t)i * P.pitch;
-        const bool row = i > 0 && i < P.ny;
-        for (int j = threadIdx.x; j <= P.nx; j += 256) {
-            double v = zero ? 0.0 : x[r + j];
-            const bool held = (!row || j == 0 || j == P.nx) && is_dirichlet(P, i, j);
-            if (held) v = dirichlet_value(P, i, j);
-            if (held || zero) x[r + j] = v;
-            u[r + j] = v;
+        for (int j = threadIdx.x; j <= P.nx; j += 256) u[r + j] = x[r + j];
+    }
+}
+
+// A solve's start: the iterate takes the wall values on held nodes, and zero
+// elsewhere where no solution is kept.
+__global__ __launch_bounds__(256) void k_fast_start(const FastJob* __restrict__ jobs, int njobs,
+                                                    const LevelProb* __restrict__ probs, double* __restrict__ x,
+                                                    const CgState* __restrict__ st)
+{
+    const int t = swizzled_block();
+    if (t >= njobs) return;
+    const FastJob job = jobs[t];
+    const LevelProb& P = probs[job.prob];
+    const bool kept = st[P.prob].have_prev != 0;
+    for (int w = 0; w < 2; ++w) {
+        const int i = 2 * job.at + w;
+        if (i > P.ny) break;
+        const int64_t r = P.origin + (int64_t)i * P.pitch;
+        const bool wall = (i == 0 && (P.dmask & (1 << kBottom))) || (i == P.ny && (P.dmask & (1 << kTop)));
+        if (kept && !wall) {
+            // two columns at most
+            const int j = threadIdx.x == 0 ? 0 : P.nx;
+            if (threadIdx.x < 2 && is_dirichlet(P, i, j)) x[r + j] = dirichlet_value(P, i, j);
+            continue;
         }
+        for (int j = threadIdx.x; j <= P.nx; j += 256)
+            x[r + j] = is_dirichlet(P, i, j) ? dirichlet_value(P, i, j) : 0.0;
     }
 }
 
@@ -859,42 +957,57 @@ __global__ __launch_bounds__(NT) void k_fast_kernel(const FastPlan* __restrict__
             v = tab[pl.ch + e];
             v.y = -v.y;
         }
-        s[pad16(k)] = v;
+        s[k] = v;
     }
     __syncthreads();
-    fft_lds<T, NT, V>(s, pl, tab);
     const T r = (T)(1.0 / pl.M);
-    for (int k = threadIdx.x; k < pl.M; k += NT) {
-        const Cx<T> v = s[pad16(k)];
-        tab[pl.hh + k] = {v.x * r, v.y * r};
-    }
+    Cx<T>* h = tab + pl.hh;
+    fft_lds<T, NT, V>(s, pl, tab, [&](int k, Cx<T> v) { h[k] = {v.x * r, v.y * r}; });
 }
 
 // ------------------------------------------------------------ host: which batches, plans
 
-static bool smooth_factors(int n, FastPlan& pl)
+// Passes of an M-point transform: as few as factors of at most 10 allow, odd
+// and singly even radices first (their strided LDS writes spread over the
+// banks; radix 8 first would put a wave on four of them).  False where M has
+// a prime factor above 7.
+static bool smooth_factors(int M, FastPlan& pl)
 {
-    int two = 0, rest = n;
-    pl.nstages = 0;
-    while (rest % 2 == 0) {
-        rest /= 2;
-        ++two;
-    }
-    std::vector<int> f;
-    for (; two > 4 || two == 3; two -= 3) f.push_back(8);
-    for (; two > 1; two -= 2) f.push_back(4);
-    if (two) f.push_back(2);
-    for (int p : {7, 5, 3})
-        while (rest % p == 0) {
-            rest /= p;
-            f.push_back(p);
+    int c[4] = {0, 0, 0, 0}, rest = M;
+    const int primes[4] = {2, 3, 5, 7};
+    for (int k = 0; k < 4; ++k)
+        while (rest % primes[k] == 0) {
+            rest /= primes[k];
+            ++c[k];
         }
-    if (rest != 1 || (int)f.size() > kFastMaxStages) return false;
-    for (int r : f) pl.radix[pl.nstages++] = r;
+    if (rest != 1) return false;
+    int& two = c[0];
+    std::vector<int> odd, even;
+    for (; c[3]; --c[3]) odd.push_back(7);
+    for (; c[1] >= 2; c[1] -= 2) odd.push_back(9);
+    // pair fives (and a last three) with twos while that leaves the twos in
+    // eights and fours
+    for (; c[2]; --c[2]) {
+        const bool pair = two % 3 == 1 || (two > 0 && c[2] > 1) || (two % 3 == 2 && two > 2) || two == 1;
+        odd.push_back(pair && two > 0 ? (--two, 10) : 5);
+    }
+    if (c[1]) odd.push_back(two % 3 == 1 ? (--two, 6) : 3);
+    for (; two > 4 || two == 3; two -= 3) even.push_back(8);
+    for (; two > 1; two -= 2) even.push_back(4);
+    if (two) (odd.empty() ? odd : even).push_back(2);
+    std::sort(odd.rbegin(), odd.rend());
+    odd.insert(odd.end(), even.begin(), even.end());
+    if (odd.empty() || (int)odd.size() > kFastMaxStages) return false;
+    pl.nstages = 0;
+    int Ns = 1;
+    for (int r : odd) {
+        pl.pass[pl.nstages++] = FastPlan::Pass{r, M / r, Ns, M / r / Ns};
+        Ns *= r;
+    }
     return true;
 }
 
-static size_t fast_lds_bytes(int M, size_t elem) { return (size_t)(pad16(M - 1) + 1) * elem; }
+static size_t fast_lds_bytes(int M, size_t elem) { return (size_t)M * elem; }
 
 // the plan of rows of N cells, or false where they do not fit a block
 static bool make_plan(int N, size_t elem, FastPlan& pl)
@@ -904,9 +1017,17 @@ static bool make_plan(int N, size_t elem, FastPlan& pl)
     pl.n = 2 * N;
     pl.M = pl.n;
     if (!smooth_factors(pl.n, pl)) {
+        // the chirp's length: the cheapest (passes times points) up to an
+        // eighth above the least
         pl.chirp = 1;
-        pl.M = 3 * N + 1;
-        while (!smooth_factors(pl.M, pl)) ++pl.M;
+        FastPlan best{};
+        for (int M = 3 * N + 1; best.M == 0 || M <= (3 * N + 1) + (3 * N + 1) / 8; ++M) {
+            FastPlan t = pl;
+            if (!smooth_factors(M, t)) continue;
+            t.M = M;
+            if (best.M == 0 || (int64_t)t.M * t.nstages < (int64_t)best.M * best.nstages) best = t;
+        }
+        pl = best;
     }
     return pl.M <= kFastValuesWide * 1024 && (int64_t)fast_lds_bytes(pl.M, elem) <= kFastLds;
 }
@@ -943,6 +1064,7 @@ void fast_free(eq_batch* b)
         if (g) hipGraphExecDestroy(g);
     hipFree(F->d_plans);
     hipFree(F->d_probs);
+    hipFree(F->d_rows);
     hipFree(F->d_jobs);
     hipFree(F->d_lines);
     hipFree(F->d_tables);
@@ -1005,6 +1127,7 @@ static int fast_build_t(eq_batch* b, FastSolver* F)
     std::vector<FastPlan> plans;
     std::map<int, int> plan_of;
     std::vector<FastProb> fp(b->nprob);
+    std::vector<FastRows> rows9(b->nprob);
     std::vector<int> thr(b->nprob);
     int64_t tab = 0;
     int32_t pairs = 0;
@@ -1036,6 +1159,18 @@ static int fast_build_t(eq_batch* b, FastSolver* F)
         fp[p].npairs = (P.ny + 2) / 2;
         pairs += fp[p].npairs;
         rows = std::max(rows, P.ny + 1);
+        for (int ci = 0; ci < 3; ++ci)
+            for (int cj = 0; cj < 3; ++cj) {
+                const int i = ci == 0 ? 0 : ci == 1 ? 1 : P.ny, j = cj == 0 ? 0 : cj == 1 ? 1 : P.nx;
+                rows9[p].a[ci][cj] = row_coefs_at<double>(P, i, j);
+                double v[8] = {0, 0, 0, 0, 0, 0, 0, 0}, *o = rows9[p].b[ci][cj];
+                o[7] = rhs_row(P, i, j, 0, 0, 0, 0, 0, 0, 0);
+                for (int q = 0; q < 7; ++q) {
+                    v[q] = 1.0;
+                    o[q] = rhs_row(P, i, j, v[0], v[1], v[2], v[3], v[4], v[5], v[6]) - o[7];
+                    v[q] = 0.0;
+                }
+            }
         int nt = 64;
         while (kFastValues * nt < plans[it->second].M && nt < 2048) nt *= 2;
         thr[p] = nt; // 2048: 1024 threads of twice the values
@@ -1065,6 +1200,7 @@ static int fast_build_t(eq_batch* b, FastSolver* F)
     F->line_c = (F->line_c + 3) / 4 * 4; // whole waves
     int rc;
     if ((rc = put_table(&F->d_plans, plans, s)) || (rc = put_table(&F->d_probs, fp, s)) ||
+        (rc = put_table(&F->d_rows, rows9, s)) ||
         (rc = put_table(&F->d_jobs, jobs, s)) || (rc = put_table(&F->d_lines, lines, s)))
         return rc;
     if (hipMalloc(&F->d_tables, sizeof(Cx<T>) * tab) != hipSuccess ||
@@ -1124,14 +1260,19 @@ static void fast_chunk(eq_batch* b, int k0, int n)
     T* z = (T*)b->z;
     const double nodes = b->levels[0].nodes_all;
     const size_t lds = sizeof(double) * (40 + 2 * (size_t)F->line_c * kFastModes);
+    int32_t njobs = 0;
+    for (const FastClass& c : F->classes) njobs += c.njobs;
+    if (k0 == 0)
+        launch(b, EQ_KERNEL_SOLVE_ONCE, 0.0, k_fast_start, dim3(grid8(njobs)), dim3(256), 0, s,
+               (const FastJob*)F->d_jobs, njobs, probs, b->xprev, (const CgState*)b->d_state);
     for (int k = k0; k < k0 + n; ++k) {
         for (const FastClass& c : F->classes)
             by_threads(c.threads, [&](auto t) {
                 constexpr int NT = std::min(1024, decltype(t)::value), V = decltype(t)::value / NT * kFastValues;
                 launch(b, EQ_KERNEL_STENCIL64, c.nodes * (16.0 + sizeof(T)), k_fast_forward<T, NT, V>, dim3(grid8(c.njobs)),
                        dim3(NT), c.lds, s, (const FastJob*)F->d_jobs + c.job0, c.njobs, probs,
-                       (const FastProb*)F->d_probs, (const FastPlan*)F->d_plans, tab, (const double*)b->u,
-                       (const double*)b->xprev, z, F->d_partial, b->d_state, k, k == k0 ? 1 : 0);
+                       (const FastProb*)F->d_probs, (const FastRows*)F->d_rows, (const FastPlan*)F->d_plans, tab,
+                       (const double*)b->u, (const double*)b->xprev, z, F->d_partial, b->d_state, k, k == k0 ? 1 : 0);
             });
         const dim3 lg(grid8(F->nline)), lb(F->line_c * kFastModes);
         auto lines = [&](auto kern) {
@@ -1150,16 +1291,14 @@ static void fast_chunk(eq_batch* b, int k0, int n)
                 launch(b, EQ_KERNEL_CG_UPDATE, c.nodes * (16.0 + sizeof(T)), k_fast_backward<T, NT, V>,
                        dim3(grid8(c.njobs)), dim3(NT), c.lds, s, (const FastJob*)F->d_jobs + c.job0, c.njobs, probs,
                        (const FastProb*)F->d_probs, (const FastPlan*)F->d_plans, tab, (const T*)z, b->xprev,
-                       (const CgState*)b->d_state, k);
+                       (const CgState*)b->d_state);
             });
     }
-    int32_t njobs = 0;
-    for (const FastClass& c : F->classes) njobs += c.njobs;
     launch(b, EQ_KERNEL_SOLVE_ONCE, nodes * 16.0, k_fast_check, dim3(grid8(njobs)), dim3(256), 0, s,
-           (const FastJob*)F->d_jobs, njobs, probs, (const FastProb*)F->d_probs, (const double*)b->u,
-           (const double*)b->xprev, F->d_partial, (const CgState*)b->d_state);
+           (const FastJob*)F->d_jobs, njobs, probs, (const FastProb*)F->d_probs, (const FastRows*)F->d_rows,
+           (const double*)b->u, (const double*)b->xprev, F->d_partial, (const CgState*)b->d_state);
     launch(b, EQ_KERNEL_SOLVE_ONCE, nodes * 16.0, k_fast_commit, dim3(grid8(njobs)), dim3(256), 0, s,
-           (const FastJob*)F->d_jobs, njobs, probs, (const FastProb*)F->d_probs, b->u, b->xprev,
+           (const FastJob*)F->d_jobs, njobs, probs, (const FastProb*)F->d_probs, b->u, (const double*)b->xprev,
            (const double*)F->d_partial, b->d_state, k0 + n);
 }
 

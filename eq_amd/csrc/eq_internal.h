@@ -65,9 +65,8 @@ struct CgState {
     int32_t extrap;         // extrapolation allowed (solver setting)
     // BiCGStab: rho = (r^, r), omega, and the pieces of omega
     double rho, omega, ts, tt;
-    // fast direct solver: applications when the problem stopped; its iterate
-    // is still the zero it started from
-    int32_t fast_iter, fast_zero;
+    int32_t fast_iter;      // fast direct solver: applications when the problem stopped
+    int32_t pad_;
 };
 
 struct FastSolver; // eq_fast.hip
