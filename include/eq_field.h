@@ -310,9 +310,11 @@ int eq_batch_couple_traps_dev(eq_batch* b, int32_t trap0, int32_t ntraps, const 
  * earlier cell's deposit), then q = a + b*e is added as q/|S_c| on S_c -- the
  * reference's read -> compute -> write order inside one step
  * (src/abm/eQabm.cpp:384-405).  a, b, sampled: nc x nspecies (device); cells and
- * offsets as eq_batch_couple_traps_dev.  One workgroup per trap walks its cells
- * in order, so a trap's cells are a sequential chain: use the q-upfront entry
- * points when the amounts do not depend on the sample. */
+ * offsets as eq_batch_couple_traps_dev.  The samples are solved for through the
+ * cells' overlaps and the amounts then deposited as the q-upfront entry points
+ * do (those are cheaper when the amounts do not depend on the sample); where a
+ * cell overlaps more than 32 earlier ones, one workgroup per trap walks its
+ * cells in order. */
 int eq_batch_couple_affine_dev(eq_batch* b, int32_t trap0, int32_t ntraps, const int64_t* cell_offsets,
                                const eq_cell* d_cells, double npm, const double* d_a, const double* d_b,
                                double* d_sampled, int32_t* d_counts);
