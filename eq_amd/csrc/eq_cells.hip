@@ -961,8 +961,18 @@ static int couple_impl(eq_batch* b, int32_t t0, int32_t ntr, const int64_t* cell
     // the affine coupling's samples before the call, amounts and overlap rows
     const size_t amount_bytes = d_b ? align256(sizeof(double) * (size_t)nc * ns) : 0;
     const size_t ov_bytes = d_b ? align256(sizeof(uint2) * (size_t)nc * kOverlaps) : 0;
-    const size_t need = head + 5 * pb + align256(sizeof(double) * (size_t)total * ns) + align256(sort_bytes) +
-                        2 * amount_bytes + ov_bytes + (d_b ? align256(sizeof(int32_t) * (size_t)nc) : 0);
+    auto need_of = [&](size_t slots, size_t sort) {
+        return head + 5 * align256(sizeof(uint32_t) * slots) + align256(sizeof(double) * slots * ns) + align256(sort) +
+               2 * amount_bytes + ov_bytes + (d_b ? align256(sizeof(int32_t) * (size_t)nc) : 0);
+    };
+    size_t need = need_of((size_t)total, sort_bytes);
+    if (!fixed && !sized) {
+        // the next call of this size finds its room: it need not allocate
+        size_t sort = 0;
+        EQ_HIP(rocprim::radix_sort_pairs(nullptr, sort, (const uint32_t*)nullptr, (uint32_t*)nullptr,
+                                         (const uint32_t*)nullptr, (uint32_t*)nullptr, (size_t)b->pair_cap, 0, 32, s));
+        need = std::max(need, need_of((size_t)b->pair_cap, sort));
+    }
     if (fixed) {
         if (need > fixed->cap) return too_big(need); // nothing written outside the scratch yet
     } else if (need > b->cell_scratch_bytes) {
