@@ -554,6 +554,9 @@ __global__ __launch_bounds__(256) void k_cell_sample(const CellGeo* __restrict__
     }
 }
 
+// a host call's device staging larger than this (2.5 M cells) is given back at its end
+constexpr size_t kCoupleStageKept = (size_t)256 << 20;
+
 static size_t align256(size_t v) { return (v + 255) & ~(size_t)255; }
 
 // The coupling of a cell whose amount depends on its own sample, q = a + b e
@@ -1180,30 +1183,39 @@ int eq_batch_couple(eq_batch* b, int32_t trap, const eq_cell* cells, size_t nc, 
     const int ns = b->nspecies;
     const size_t cb = sizeof(eq_cell) * nc, qb = sizeof(double) * nc * ns, sb = sizeof(double) * nc * ns,
                  kb = sizeof(int32_t) * nc;
-    char* buf = nullptr;
+    // (allocated and freed on each call, this buffer took half of it)
     const size_t tot = align256(cb) + align256(qb) + align256(sb) + align256(kb);
-    if (hipMalloc((void**)&buf, tot) != hipSuccess) return set_error(EQ_ERR_NOMEM, "couple staging");
+    char* buf = (char*)b->couple_stage;
+    if (tot > b->couple_stage_bytes) {
+        hipStreamSynchronize(b->stream);
+        hipFree(b->couple_stage);
+        b->couple_stage = nullptr;
+        b->couple_stage_bytes = 0;
+        if (hipMalloc((void**)&buf, tot + tot / 4) != hipSuccess) return set_error(EQ_ERR_NOMEM, "couple staging");
+        b->couple_stage = buf;
+        b->couple_stage_bytes = tot + tot / 4;
+    }
     eq_cell* dc = (eq_cell*)buf;
     double* dq = (double*)(buf + align256(cb));
     double* ds = (double*)(buf + align256(cb) + align256(qb));
     int32_t* dk = (int32_t*)(buf + align256(cb) + align256(qb) + align256(sb));
-    int rc = EQ_OK;
     hipStream_t s = b->stream;
-    if (hipMemcpyAsync(dc, cells, cb, hipMemcpyHostToDevice, s) != hipSuccess ||
-        (q && hipMemcpyAsync(dq, q, qb, hipMemcpyHostToDevice, s) != hipSuccess)) {
-        rc = set_error(EQ_ERR_HIP, "couple upload");
-    } else if (!q) {
+    int rc = rows_from_host(b, (double*)dc, 1024, 1024, cells, cb, nullptr);
+    if (rc == EQ_OK && q)
+        rc = rows_from_host(b, dq, 1024, 1024, q, qb, nullptr);
+    else if (rc == EQ_OK)
         hipMemsetAsync(dq, 0, qb, s);
-    }
     const int64_t off[2] = {0, (int64_t)nc};
     if (rc == EQ_OK)
         rc = couple_impl(b, trap, 1, off, dc, npm, dq, sampled ? ds : nullptr, counts ? dk : nullptr, flags);
-    if (rc == EQ_OK && sampled && hipMemcpyAsync(sampled, ds, sb, hipMemcpyDeviceToHost, s) != hipSuccess)
-        rc = set_error(EQ_ERR_HIP, "couple download");
-    if (rc == EQ_OK && counts && hipMemcpyAsync(counts, dk, kb, hipMemcpyDeviceToHost, s) != hipSuccess)
-        rc = set_error(EQ_ERR_HIP, "couple download");
+    if (rc == EQ_OK && sampled) rc = rows_to_host(b, ds, 1024, 1024, sampled, sb);
+    if (rc == EQ_OK && counts) rc = rows_to_host(b, (const double*)dk, 1024, 1024, counts, kb);
     hipStreamSynchronize(s);
-    hipFree(buf);
+    if (b->couple_stage_bytes > kCoupleStageKept) {
+        hipFree(b->couple_stage);
+        b->couple_stage = nullptr;
+        b->couple_stage_bytes = 0;
+    }
     return rc;
 }
 

@@ -342,15 +342,15 @@ int eq_batch_channel_values(eq_batch* b, int32_t prob, double* top, double* bott
     if (!b) return set_error(EQ_ERR_INVALID, "NULL batch");
     if (prob < 0 || prob >= b->nprob) return set_error(EQ_ERR_INVALID, "problem index out of range");
     hipSetDevice(b->device);
-    EQ_HIP(hipStreamSynchronize(b->stream));
     const LevelProb& P = b->levels[0].probs[prob];
     double* out[2] = {top, bottom};
     for (int side = 0; side < 2; ++side) {
         if (!out[side]) continue;
         if ((int)b->chan_desc.size() <= prob || b->chan_desc[prob][side].substeps == 0)
             return set_error(EQ_ERR_INVALID, "no channel on that side");
-        EQ_HIP(hipMemcpy(out[side], b->wall_vals[prob][side == 0 ? kTop : kBottom], sizeof(double) * (P.nx + 1),
-                         hipMemcpyDeviceToHost));
+        const int rc = rows_to_host(b, b->wall_vals[prob][side == 0 ? kTop : kBottom], 1024, 1024, out[side],
+                                    sizeof(double) * (P.nx + 1));
+        if (rc) return rc;
     }
     return EQ_OK;
 }

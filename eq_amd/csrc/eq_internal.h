@@ -274,6 +274,13 @@ struct eq_batch {
     std::vector<eqk::WellDev> wells;
     eqk::WellDev* d_wells = nullptr;
     int32_t d_wells_cap = 0;
+    // pinned staging of host arrays (allocated on first use) and the events
+    // behind the last kernel that read or wrote each
+    double* stage[2] = {nullptr, nullptr};
+    hipEvent_t stage_ev[2] = {nullptr, nullptr};
+    // device staging of the host-array coupling (kept up to kCoupleStageKept)
+    void* couple_stage = nullptr;
+    size_t couple_stage_bytes = 0;
     // algorithmic traffic: launches add to *acct_to, which is `acct` except
     // while a graph is captured (then the graph's own count, added to `acct`
     // at every replay)
@@ -311,6 +318,11 @@ int refresh_cell_tensors(eq_batch* b);
 int set_trap_tensor(eq_batch* b, int trap, double Dx, double Dy, int on);
 // the coupling's tables and the fixed scratch's device address (at batch creation)
 int init_coupling(eq_batch* b);
+// host arrays in and out (eq_transfer.hip): to rows of w doubles with pitch p,
+// back, and the staging released
+int rows_from_host(eq_batch* b, double* rows, int64_t w, int64_t p, const void* src, size_t bytes, int32_t* restart);
+int rows_to_host(eq_batch* b, const double* rows, int64_t w, int64_t p, void* dst, size_t bytes);
+void free_stage(eq_batch* b);
 // the fast direct solver (eq_fast.hip): plans at batch creation; whether the
 // next step takes it; one solve (handled = false: the multigrid solver has to
 // go on); graphs and plans dropped

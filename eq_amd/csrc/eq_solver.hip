@@ -4722,6 +4722,7 @@ void eq_batch_destroy(eq_batch* b)
     hipFree(b->flux_out);
     hipFree(b->d_field_ptrs);
     hipFree(b->cell_scratch);
+    hipFree(b->couple_stage);
     hipFree(b->d_wells);
     hipFree(b->d_tens64);
     hipFree(b->d_tens32);
@@ -4729,6 +4730,7 @@ void eq_batch_destroy(eq_batch* b)
     hipFree(b->d_inv_jobs);
     hipFree(b->inv_scratch);
     free_channels(b);
+    free_stage(b);
     fast_free(b);
     hipFree(b->d_cell_traps);
     hipFree(b->d_cell_off);
@@ -4765,62 +4767,6 @@ int eq_batch_sync(eq_batch* b)
 {
     if (!b) return set_error(EQ_ERR_INVALID, "NULL batch");
     EQ_HIP(hipStreamSynchronize(b->stream));
-    return EQ_OK;
-}
-
-static int copy_field(eq_batch* b, int32_t prob, const double* src, double* dst, size_t n, hipMemcpyKind kind,
-                      bool sync)
-{
-    if (!b) return set_error(EQ_ERR_INVALID, "NULL batch");
-    if (prob < 0 || prob >= b->nprob) return set_error(EQ_ERR_INVALID, "problem index out of range");
-    const LevelProb& P = b->levels[0].probs[prob];
-    const size_t nw = (size_t)P.nx + 1, nh = (size_t)P.ny + 1;
-    if (n != nw * nh) return set_error(EQ_ERR_INVALID, "length must be (nx+1)*(ny+1)");
-    if (!src && !dst) return set_error(EQ_ERR_INVALID, "NULL data");
-    double* dev = b->u + P.origin;
-    const bool to_dev = (kind == hipMemcpyHostToDevice) || (dst == nullptr);
-    if (to_dev) {
-        // a new state from the host: the kept solution is no starting point for it
-        EQ_HIP(hipMemsetAsync(&b->d_state[prob].have_prev, 0, 2 * sizeof(int32_t), b->stream)); // and have_prev2
-        EQ_HIP(hipMemcpy2DAsync(dev, sizeof(double) * P.pitch, src, sizeof(double) * nw, sizeof(double) * nw, nh,
-                                kind, b->stream));
-    } else {
-        EQ_HIP(hipMemcpy2DAsync(dst, sizeof(double) * nw, dev, sizeof(double) * P.pitch, sizeof(double) * nw, nh,
-                                kind, b->stream));
-    }
-    if (sync) EQ_HIP(hipStreamSynchronize(b->stream));
-    return EQ_OK;
-}
-
-int eq_batch_upload(eq_batch* b, int32_t prob, const double* u, size_t n)
-{
-    if (!u) return set_error(EQ_ERR_INVALID, "NULL data");
-    return copy_field(b, prob, u, nullptr, n, hipMemcpyHostToDevice, true);
-}
-
-int eq_batch_download(eq_batch* b, int32_t prob, double* u, size_t n)
-{
-    if (!u) return set_error(EQ_ERR_INVALID, "NULL data");
-    return copy_field(b, prob, nullptr, u, n, hipMemcpyDeviceToHost, true);
-}
-
-int eq_batch_upload_dev(eq_batch* b, int32_t prob, const double* d_u, size_t n)
-{
-    if (!d_u) return set_error(EQ_ERR_INVALID, "NULL data");
-    return copy_field(b, prob, d_u, nullptr, n, hipMemcpyDeviceToDevice, false);
-}
-
-int eq_batch_download_dev(eq_batch* b, int32_t prob, double* d_u, size_t n)
-{
-    if (!d_u) return set_error(EQ_ERR_INVALID, "NULL data");
-    // device-to-device: the destination is natural order
-    if (!b) return set_error(EQ_ERR_INVALID, "NULL batch");
-    if (prob < 0 || prob >= b->nprob) return set_error(EQ_ERR_INVALID, "problem index out of range");
-    const LevelProb& P = b->levels[0].probs[prob];
-    const size_t nw = (size_t)P.nx + 1, nh = (size_t)P.ny + 1;
-    if (n != nw * nh) return set_error(EQ_ERR_INVALID, "length must be (nx+1)*(ny+1)");
-    EQ_HIP(hipMemcpy2DAsync(d_u, sizeof(double) * nw, b->u + P.origin, sizeof(double) * P.pitch,
-                            sizeof(double) * nw, nh, hipMemcpyDeviceToDevice, b->stream));
     return EQ_OK;
 }
 
