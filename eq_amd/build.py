@@ -15,8 +15,9 @@ ROOT = os.path.dirname(HERE)
 CSRC = os.path.join(HERE, "csrc")
 LIB_DIR = os.path.join(HERE, "lib")
 LIB = os.path.join(LIB_DIR, "libeq_field.so")
-SOURCES = ["eq_solver.hip", "eq_fast.hip", "eq_cells.hip", "eq_channels.hip", "eq_transfer.hip"]
-HEADERS = ["eq_common.h", "eq_internal.h"]
+SOURCES = ["eq_solver.hip", "eq_fast.hip", "eq_fast_f32.hip", "eq_fast_f32_general.hip",
+           "eq_fast_f64.hip", "eq_fast_f64_general.hip", "eq_cells.hip", "eq_channels.hip", "eq_transfer.hip"]
+HEADERS = ["eq_common.h", "eq_internal.h", "eq_fast.h", "eq_fast_launch.h"]
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 FLAGS = [

@@ -293,6 +293,8 @@ struct eq_batch {
     double** d_tens64 = nullptr;
     float** d_tens32 = nullptr;
     std::vector<int32_t> cell_tensor_traps;
+    std::vector<std::array<double, 2>> tens_bounds; // per problem: least and largest eigenvalue of its tensor field
+    bool coarse_tensors_stale = false; // the finest level's tensors have still to be carried to the coarse levels
     std::vector<eqk::InvJob> inv_jobs;
     eqk::InvJob* d_inv_jobs = nullptr;
     double* inv_scratch = nullptr;
@@ -327,6 +329,7 @@ void free_stage(eq_batch* b);
 // next step takes it; one solve (handled = false: the multigrid solver has to
 // go on); graphs and plans dropped
 int fast_build(eq_batch* b);
+int fast_refresh(eq_batch* b); // after a change of tensor fields or velocities
 bool fast_applies(const eq_batch* b);
 int fast_solve(eq_batch* b, bool profiling, bool* handled);
 void fast_drop_graphs(eq_batch* b);

@@ -4424,6 +4424,10 @@ static int solve_ir(eq_batch* b, eq_step_stats* stats)
 }
 
 // precision of the multigrid x whether any problem carries a tensor field
+namespace eqk {
+template <typename T>
+static int refresh_cell_tensors_t(eq_batch* b);
+}
 static int run_multigrid(eq_batch* b, eq_step_stats* stats);
 
 // The fast direct solver where it applies.  Where it gives up (a residual
@@ -4466,6 +4470,11 @@ static int run_solve(eq_batch* b, eq_step_stats* stats)
 
 static int run_multigrid(eq_batch* b, eq_step_stats* stats)
 {
+    if (b->coarse_tensors_stale) {
+        b->coarse_tensors_stale = false;
+        const int rc = b->mixed ? refresh_cell_tensors_t<float>(b) : refresh_cell_tensors_t<double>(b);
+        if (rc) return rc;
+    }
     const bool bicg = b->solver.kind == EQ_SOLVER_GMG_BICGSTAB || b->solver.kind == EQ_SOLVER_MIXED_GMG_BICGSTAB;
     if (!bicg)
         for (const LevelProb& P : b->levels[0].probs)
@@ -4891,7 +4900,7 @@ static int set_tensor_impl(eq_batch* b, int32_t prob, const double* d11, const d
 
 // The kernels specialise on whether any problem has per-node rows (tensor
 // field or advection); a change of that drops the captured graphs.
-static void refresh_general(eq_batch* b)
+static int refresh_general(eq_batch* b)
 {
     bool any = false;
     for (const LevelProb& P : b->levels[0].probs) any = any || P.aniso || P.vel;
@@ -4899,6 +4908,7 @@ static void refresh_general(eq_batch* b)
         b->any_tensor = any;
         drop_graphs(b);
     }
+    return fast_refresh(b);
 }
 
 static int set_tensor_checked(eq_batch* b, int32_t prob, const double* D11, const double* D22, const double* D12,
@@ -4913,6 +4923,17 @@ static int set_tensor_checked(eq_batch* b, int32_t prob, const double* D11, cons
     if (all && P.fd) return set_error(EQ_ERR_INVALID, "the finite-difference scheme has no tensor field");
     if (all && P.vel) return set_error(EQ_ERR_INVALID, "advection and a tensor field together are not supported");
     hipSetDevice(b->device);
+    if (all) {
+        double lo = HUGE_VAL, hi = -HUGE_VAL;
+        for (size_t k = 0; k < n; ++k) {
+            const double m = 0.5 * (D11[k] + D22[k]), w = std::hypot(0.5 * (D11[k] - D22[k]), D12[k]);
+            if (!std::isfinite(m) || !std::isfinite(w)) lo = -HUGE_VAL;
+            lo = std::min(lo, m - w);
+            hi = std::max(hi, m + w);
+        }
+        b->tens_bounds.resize(b->nprob, {1.0, 1.0});
+        b->tens_bounds[prob] = {lo, hi};
+    }
     return b->mixed ? set_tensor_impl<float>(b, prob, D11, D22, D12) : set_tensor_impl<double>(b, prob, D11, D22, D12);
 }
 
@@ -4945,8 +4966,14 @@ static int refresh_cell_tensors_t(eq_batch* b)
     return EQ_OK;
 }
 
+// (the fast solver reads the finest level alone: where it takes the next step,
+// the rest waits for a multigrid solve; a captured coupling carries it all)
 int refresh_cell_tensors(eq_batch* b)
 {
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    EQ_HIP(hipStreamIsCapturing(b->stream, &cap));
+    b->coarse_tensors_stale = cap == hipStreamCaptureStatusNone && fast_applies(b);
+    if (b->coarse_tensors_stale) return EQ_OK;
     return b->mixed ? refresh_cell_tensors_t<float>(b) : refresh_cell_tensors_t<double>(b);
 }
 
@@ -4977,8 +5004,10 @@ int eq_batch_cell_tensor(eq_batch* b, int32_t trap, double Dx, double Dy, int32_
         // start from the reference's isotropic grids; this allocates the tensor
         // arrays of every level and marks the problems anisotropic
         std::vector<double> one(n, 1.0), zero(n, 0.0);
-        for (int p = p0; p < p0 + ns; ++p)
+        for (int p = p0; p < p0 + ns; ++p) {
             if ((rc = set_tensor_checked(b, p, one.data(), one.data(), zero.data(), n))) return rc;
+            b->tens_bounds[p] = {std::min({1.0, Dx, Dy}), std::max({1.0, Dx, Dy})};
+        }
     } else {
         for (int p = p0; p < p0 + ns; ++p)
             if ((rc = set_tensor_checked(b, p, nullptr, nullptr, nullptr, 0))) return rc;
@@ -5039,8 +5068,7 @@ int eq_batch_cell_tensor(eq_batch* b, int32_t trap, double Dx, double Dy, int32_
             return set_error(EQ_ERR_NOMEM, "coarsest inverse scratch");
         EQ_HIP(hipMemcpy(b->d_inv_jobs, b->inv_jobs.data(), sizeof(InvJob) * b->inv_jobs.size(), hipMemcpyHostToDevice));
     }
-    refresh_general(b);
-    return EQ_OK;
+    return refresh_general(b);
 }
 
 int eq_batch_tensor_values(eq_batch* b, int32_t prob, double* D11, double* D22, double* D12, size_t n)
@@ -5070,8 +5098,7 @@ int eq_batch_set_tensor(eq_batch* b, int32_t prob, const double* D11, const doub
 {
     int rc = set_tensor_checked(b, prob, D11, D22, D12, n);
     if (rc != EQ_OK || !b) return rc;
-    refresh_general(b);
-    return EQ_OK;
+    return refresh_general(b);
 }
 
 
@@ -5157,8 +5184,7 @@ int eq_batch_set_velocity(eq_batch* b, int32_t prob, const double* vx, size_t n)
     hipSetDevice(b->device);
     const int rc = b->mixed ? set_velocity_impl<float>(b, prob, vx) : set_velocity_impl<double>(b, prob, vx);
     if (rc) return rc;
-    refresh_general(b);
-    return EQ_OK;
+    return refresh_general(b);
 }
 
 int eq_field_set_tensor(eq_field* f, const double* D11, const double* D22, const double* D12, size_t n)
