@@ -51,6 +51,17 @@ struct FastPlan {
 struct FastProb {
     int32_t plan, ends;
     int32_t pair0, npairs;  // this problem's slots of row-pair partials
+    int64_t mode0;          // its modes' records
+};
+
+// A mode's tridiagonal inverse along y (k_fast_lines), laid out once: forming
+// it takes a thread more time than the sweeps of 16 rows do.
+struct FastMode {
+    double rho, irho; // the decay of both recursions, and 1 / rho
+    double scale;     // c and both transforms' factors
+    double a0, a1;    // A = a0 w_0 + a1 w_ny
+    double b0, b1;    // B = b0 w_ny + b1 A
+    double w, wl;     // rho to the rows of a chunk, and of the last one
 };
 
 // The rows of a problem's operator and right-hand side by place: bottom row,
@@ -83,6 +94,7 @@ struct FastSolver {
     FastRows* d_rows = nullptr;
     FastJob* d_jobs = nullptr;   // row pairs, class by class
     FastJob* d_lines = nullptr;  // mode groups
+    FastMode* d_modes = nullptr;
     void* d_tables = nullptr;
     double* d_partial = nullptr; // 2 per row pair
     // varying coefficients (tensor field, advection): per problem kChebMax

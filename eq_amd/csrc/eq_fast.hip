@@ -97,6 +97,49 @@ __device__ __forceinline__ double ipow(double a, int n)
     return r;
 }
 
+// Every mode's record.
+__global__ __launch_bounds__(256) void k_fast_modes(const LevelProb* __restrict__ probs,
+                                                    const FastProb* __restrict__ fp, FastMode* __restrict__ modes, int C)
+{
+    const LevelProb& P = probs[blockIdx.x];
+    const FastProb f = fp[blockIdx.x];
+    const int N = P.nx, ny = P.ny, rows = ny + 1, Lp = (rows + C - 1) / C;
+    const bool half = f.ends >= kEndsND;
+    for (int q = threadIdx.x; q <= N; q += 256) {
+        const double cx = cospi((half ? q + 0.5 : (double)q) / N), lx = 2.0 * (1.0 - cx);
+        double sigma, tau, k0 = 0.0, k1 = 0.0;
+        if (P.fd) {
+            sigma = P.fdm + P.fkx * lx;
+            tau = P.fky;
+            k0 = P.frob[kBottom];
+            k1 = P.frob[kTop];
+        } else {
+            const double ms = 12.0 * P.mh;
+            sigma = ms * (2.0 + cx) / 3.0 + 2.0 * P.sa * lx;
+            tau = 2.0 * P.sb - ms * (1.0 + cx) / 12.0;
+            k0 = P.rob[kBottom] * 2.0 * (2.0 + cx) / 3.0;
+            k1 = P.rob[kTop] * 2.0 * (2.0 + cx) / 3.0;
+        }
+        const double sh = sigma / tau;
+        const double rho = 1.0 / (1.0 + 0.5 * sh + sqrt(sh + 0.25 * sh * sh));
+        const double del = 1.0 / rho - rho;
+        const double R0 = (P.dmask & (1 << kBottom)) ? -1.0 : (del - k0 / tau) / (del + k0 / tau);
+        const double R1 = (P.dmask & (1 << kTop)) ? -1.0 : (del - k1 / tau) / (del + k1 / tau);
+        const double pn = ipow(rho, ny), den = 1.0 - R0 * R1 * pn * pn;
+        FastMode m;
+        m.rho = rho;
+        m.irho = 1.0 / rho;
+        m.scale = 1.0 / (tau * del * 2.0 * N); // both transforms' factors with it
+        m.a0 = R0 / den;
+        m.a1 = R0 * R1 * pn / den;
+        m.b0 = R1;
+        m.b1 = R1 * pn;
+        m.w = ipow(rho, Lp);
+        m.wl = ipow(rho, rows - (rows - 1) / Lp * Lp);
+        modes[f.mode0 + q] = m;
+    }
+}
+
 // The tridiagonal solves along y, 16 modes a block, C chunks of rows each in
 // the registers of one thread.  Per mode the matrix is (sigma + tau Lambda)
 // with Lambda the second difference: its inverse on the whole line is
@@ -106,14 +149,18 @@ __device__ __forceinline__ double ipow(double a, int n)
 // R = 1 for a closed wall, -1 for a held one and between for Robin.  All
 // recursions decay, in FP64.  First every block takes its problem's residual
 // norm from the row pairs' sums and stops where it converged.
+// Bound by latency (one block a CU at 2000x1000, 2 species): the carries go
+// through four chunks of a wave by shuffles, then once through LDS; walked
+// chunk by chunk by one thread a mode, and with the modes' constants formed in
+// every thread, it took 21.7 us, now 16.6 (32 MB: 6 us); 800x400 14.3 -> 11.1.
 template <typename T, int L>
 __global__ void k_fast_lines(const FastJob* __restrict__ jobs, int njobs, const LevelProb* __restrict__ probs,
-                             const FastProb* __restrict__ fp, T* __restrict__ io, const double* __restrict__ partial,
-                             CgState* st, const int32_t* __restrict__ extra, int32_t* met_at, int k)
+                             const FastProb* __restrict__ fp, const FastMode* __restrict__ modes, T* __restrict__ io,
+                             const double* __restrict__ partial, CgState* st, const int32_t* __restrict__ extra,
+                             int32_t* met_at, int k)
 {
-    extern __shared__ char lds_raw[];
-    double* red = (double*)lds_raw;            // 32 doubles of sums, then the flag
-    double* carry = red + 40;                  // [2][C][16] chunk ends
+    __shared__ double red[40];                  // 32 doubles of sums, then the flags
+    __shared__ double tot[2][16][kFastModes];   // the waves' totals, up and down
     const int t = swizzled_block();
     if (t >= njobs) return;
     const FastJob job = jobs[t];
@@ -131,6 +178,7 @@ __global__ void k_fast_lines(const FastJob* __restrict__ jobs, int njobs, const 
     T v[L];
 #pragma unroll
     for (int l = 0; l < L; ++l) v[l] = (on && l < nl) ? col[(int64_t)l * P.pitch] : (T)0;
+    const FastMode M = modes[f.mode0 + min(q, N)];
     if (threadIdx.x == 0) {
         ((int*)(red + 36))[0] = k > 0 ? cs.done : 0;
         ((int*)(red + 36))[1] = k > 0 ? met_at[P.prob] : -1;
@@ -154,28 +202,7 @@ __global__ void k_fast_lines(const FastJob* __restrict__ jobs, int njobs, const 
         }
     }
     if (stop) return;
-    // the mode's matrix
-    const bool half = f.ends >= kEndsND;
-    const double cx = cospi((half ? q + 0.5 : (double)q) / N), lx = 2.0 * (1.0 - cx);
-    double sigma, tau, k0 = 0.0, k1 = 0.0;
-    if (P.fd) {
-        sigma = P.fdm + P.fkx * lx;
-        tau = P.fky;
-        k0 = P.frob[kBottom];
-        k1 = P.frob[kTop];
-    } else {
-        const double ms = 12.0 * P.mh;
-        sigma = ms * (2.0 + cx) / 3.0 + 2.0 * P.sa * lx;
-        tau = 2.0 * P.sb - ms * (1.0 + cx) / 12.0;
-        k0 = P.rob[kBottom] * 2.0 * (2.0 + cx) / 3.0;
-        k1 = P.rob[kTop] * 2.0 * (2.0 + cx) / 3.0;
-    }
-    const double sh = sigma / tau;
-    const double rho = 1.0 / (1.0 + 0.5 * sh + sqrt(sh + 0.25 * sh * sh));
-    const double del = 1.0 / rho - rho;
-    const double R0 = (P.dmask & (1 << kBottom)) ? -1.0 : (del - k0 / tau) / (del + k0 / tau);
-    const double R1 = (P.dmask & (1 << kTop)) ? -1.0 : (del - k1 / tau) / (del + k1 / tau);
-    const double scale = 1.0 / (tau * del * 2.0 * N); // both transforms' factors with it
+    const double rho = M.rho;
     // chunk ends from zero carries: F at the chunk's last row, G before its first
     double F = 0.0, G = 0.0;
 #pragma unroll
@@ -184,60 +211,44 @@ __global__ void k_fast_lines(const FastJob* __restrict__ jobs, int njobs, const 
 #pragma unroll
     for (int l = L - 1; l >= 0; --l)
         if (l < nl) G = rho * (G + (double)v[l]);
-    double* cF = carry + c * kFastModes + m;
-    double* cG = cF + C * kFastModes;
-    *cF = F;
-    *cG = G;
-    __syncthreads();
-    // carries across the chunks: a thread per mode up, another down
-    if (threadIdx.x < 2 * kFastModes) {
-        const int mm = threadIdx.x & (kFastModes - 1);
-        const double w = ipow(rho, Lp); // (a thread's own mode is mm)
-        double* p = carry + mm + (threadIdx.x < kFastModes ? 0 : C * kFastModes);
-        double in = 0.0;
-        if (threadIdx.x < kFastModes) {
-            for (int e = 0; e < C; ++e) {
-                const double own = p[e * kFastModes];
-                p[e * kFastModes] = in;
-                in = w * in + own;
-            }
-        } else {
-            for (int e = C - 1; e >= 0; --e) {
-                const double own = p[e * kFastModes];
-                p[e * kFastModes] = in;
-                in = w * in + own; // rows past the last are zero: their chunk's power only scales zero
-            }
-        }
+    // carries across the chunks: inclusive over the wave's four, then the waves.
+    // (Rows past the last are zero, so the powers there only scale zero.)
+    const int w = threadIdx.x >> 6, nw = blockDim.x >> 6, cl = (threadIdx.x & 63) / kFastModes;
+    const double w1 = M.w, w2 = w1 * w1, w4 = w2 * w2;
+    double Fi = F, Gi = G;
+    {
+        double up = __shfl_up(Fi, kFastModes, 64), dn = __shfl_down(Gi, kFastModes, 64);
+        if (cl >= 1) Fi += w1 * up;
+        if (cl <= 2) Gi += w1 * dn;
+        up = __shfl_up(Fi, 2 * kFastModes, 64);
+        dn = __shfl_down(Gi, 2 * kFastModes, 64);
+        if (cl >= 2) Fi += w2 * up;
+        if (cl <= 1) Gi += w2 * dn;
     }
+    if (cl == 3) tot[0][w][m] = Fi;
+    if (cl == 0) tot[1][w][m] = Gi;
     __syncthreads();
-    // w on the whole line at the two walls (in units of c): bottom f_0 + G_0,
-    // top F_ny; their threads publish them
-    double* ends = red; // [2][16]
-    F = *cF;
-    G = *cG;
-    if (a == 0) {
-        double g = G;
-#pragma unroll
-        for (int l = L - 1; l >= 1; --l)
-            if (l < nl) g = rho * (g + (double)v[l]);
-        ends[m] = (double)v[0] + g;
-    }
-    if (nl > 0 && a + nl == rows) {
-        double e = F;
-#pragma unroll
-        for (int l = 0; l < L; ++l)
-            if (l < nl) e = rho * e + (double)v[l];
-        ends[kFastModes + m] = e;
+    double fin = 0.0, gin = 0.0; // at the wave's edges
+    for (int e = 0; e < w; ++e) fin = w4 * fin + tot[0][e][m];
+    for (int e = nw - 1; e > w; --e) gin = w4 * gin + tot[1][e][m];
+    {
+        const double up = __shfl_up(Fi, kFastModes, 64), dn = __shfl_down(Gi, kFastModes, 64);
+        const double own = F, owng = G, wc[4] = {1.0, w1, w2, w1 * w2};
+        F = cl == 0 ? fin : up + (cl == 1 ? wc[1] : cl == 2 ? wc[2] : wc[3]) * fin;
+        G = cl == 3 ? gin : dn + (cl == 2 ? wc[1] : cl == 1 ? wc[2] : wc[3]) * gin;
+        // w on the whole line at the two walls (in units of c): bottom f_0 +
+        // G_0, top F_ny; their threads publish them
+        if (c == 0) red[m] = (owng + w1 * G) * M.irho;
+        if (nl > 0 && a + nl == rows) red[kFastModes + m] = own + M.wl * F;
     }
     __syncthreads();
     if (!on || nl == 0) return;
-    const double pn = ipow(rho, ny);
-    const double w0 = ends[m], wn = ends[kFastModes + m];
-    const double A = R0 * (w0 + pn * R1 * wn) / (1.0 - R0 * R1 * pn * pn);
-    const double B = R1 * (wn + pn * A);
+    const double w0 = red[m], wn = red[kFastModes + m];
+    const double A = M.a0 * w0 + M.a1 * wn, B = M.b0 * wn + M.b1 * A;
     // the walls' terms ride on the recursions' carries: F gets A rho^i, G gets B rho^(ny - i)
-    F += A * ipow(rho, a) / rho;                     // at row a - 1
-    G += B * ipow(rho, rows - (a + nl));             // at the chunk's last row
+    const int last = (rows - 1) / Lp;
+    F += A * ipow(w1, c) * M.irho;                              // at row a - 1
+    G += c == last ? B : B * ipow(w1, last - c - 1) * M.wl;     // at the chunk's last row
     // both directions through the registers: G_i kept, then F_i + G_i
     T g[L];
 #pragma unroll
@@ -250,7 +261,7 @@ __global__ void k_fast_lines(const FastJob* __restrict__ jobs, int njobs, const 
     for (int l = 0; l < L; ++l)
         if (l < nl) {
             F = rho * F + (double)v[l];
-            col[(int64_t)l * P.pitch] = (T)(scale * (F + (double)g[l]));
+            col[(int64_t)l * P.pitch] = (T)(M.scale * (F + (double)g[l]));
         }
 }
 
@@ -479,6 +490,7 @@ void fast_free(eq_batch* b)
     hipFree(F->d_rows);
     hipFree(F->d_jobs);
     hipFree(F->d_lines);
+    hipFree(F->d_modes);
     hipFree(F->d_tables);
     hipFree(F->d_partial);
     hipFree(F->d_cheb);
@@ -517,6 +529,7 @@ static int fast_build_t(eq_batch* b, FastSolver* F)
     std::vector<int> thr(b->nprob);
     int64_t tab = 0;
     int32_t pairs = 0;
+    int64_t modes = 0;
     int rows = 0, mmax = 1;
     for (int p = 0; p < b->nprob; ++p) {
         const LevelProb& P = b->levels[0].probs[p];
@@ -544,6 +557,8 @@ static int fast_build_t(eq_batch* b, FastSolver* F)
         fp[p].pair0 = pairs;
         fp[p].npairs = (P.ny + 2) / 2;
         pairs += fp[p].npairs;
+        fp[p].mode0 = modes;
+        modes += P.nx + 1;
         rows = std::max(rows, P.ny + 1);
         for (int ci = 0; ci < 3; ++ci)
             for (int cj = 0; cj < 3; ++cj) {
@@ -591,10 +606,13 @@ static int fast_build_t(eq_batch* b, FastSolver* F)
         return rc;
     if (hipMalloc(&F->d_tables, sizeof(Cx<T>) * tab) != hipSuccess ||
         hipMalloc((void**)&F->d_partial, sizeof(double) * 2 * pairs) != hipSuccess ||
+        hipMalloc((void**)&F->d_modes, sizeof(FastMode) * modes) != hipSuccess ||
         hipMalloc((void**)&F->d_extra, sizeof(int32_t) * b->nprob) != hipSuccess ||
         hipMalloc((void**)&F->d_met, sizeof(int32_t) * b->nprob) != hipSuccess)
         return set_error(EQ_ERR_NOMEM, "fast solver tables");
     EQ_HIP(hipMemsetAsync(F->d_extra, 0, sizeof(int32_t) * b->nprob, s));
+    hipLaunchKernelGGL(k_fast_modes, dim3(b->nprob), dim3(256), 0, s, (const LevelProb*)b->levels[0].d_probs,
+                       (const FastProb*)F->d_probs, F->d_modes, (int)F->line_c);
     const int np = (int)plans.size();
     hipLaunchKernelGGL(k_fast_tables<T>, dim3(np, 4), dim3(256), 0, s, F->d_plans, (Cx<T>*)F->d_tables);
     if (mmax > 1) {
@@ -729,7 +747,6 @@ static void fast_chunk(eq_batch* b, int k0, int n)
     const LevelProb* probs = b->levels[0].d_probs;
     T* z = (T*)b->z;
     const double nodes = b->levels[0].nodes_all;
-    const size_t lds = sizeof(double) * (40 + 2 * (size_t)F->line_c * kFastModes);
     int32_t njobs = 0;
     for (const FastClass& c : F->classes) njobs += c.njobs;
     if (k0 == 0)
@@ -739,8 +756,8 @@ static void fast_chunk(eq_batch* b, int k0, int n)
         fast_forward<T, GEN>(b, k, k == k0);
         const dim3 lg(grid8(F->nline)), lb(F->line_c * kFastModes);
         auto lines = [&](auto kern) {
-            launch(b, EQ_KERNEL_BOTTOM, nodes * 2 * sizeof(T), kern, lg, lb, lds, s, (const FastJob*)F->d_lines, F->nline,
-                   probs, (const FastProb*)F->d_probs, z, (const double*)F->d_partial, b->d_state, (const int32_t*)F->d_extra, F->d_met, k);
+            launch(b, EQ_KERNEL_BOTTOM, nodes * 2 * sizeof(T), kern, lg, lb, 0, s, (const FastJob*)F->d_lines, F->nline,
+                   probs, (const FastProb*)F->d_probs, (const FastMode*)F->d_modes, z, (const double*)F->d_partial, b->d_state, (const int32_t*)F->d_extra, F->d_met, k);
         };
         if (F->line_rows <= 1024)
             lines(k_fast_lines<T, 16>);
