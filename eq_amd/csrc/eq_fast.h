@@ -104,6 +104,11 @@ struct FastSolver {
     int32_t* d_extra = nullptr;  // per problem: applications after the tolerance is met,
     int32_t* d_met = nullptr;    // and where it first was (-1: not yet)
     bool general_ok = false;
+    // tensor fields: the stiffness weights of every node to its W, S and SW
+    // neighbour (three arrays of level 0's layout, zero in the frame), formed
+    // anew by each solve
+    double* d_stiff = nullptr;
+    int64_t stiff_stride = 0;
     int recent[2][4] = {{3, 3, 3, 3}, {3, 3, 3, 3}}; // application counts of the last solves, constant and varying
     int at[2] = {0, 0};
     static constexpr int kGraphs = 49;
@@ -424,6 +429,16 @@ struct PairWindow { // rows i0-1 .. i0+2 of column j, and of its neighbours as f
     {
         return row_apply<true>(r, m[k + 1], w[k + 1], e[k], m[k], m[k + 2], w[k], e[k + 1]);
     }
+    // a row off the walls from its stiffness weights: s points at the row's
+    // node in the weights to W, to S and to SW (the others are theirs)
+    __device__ __forceinline__ double apply_stiff(double mc, double mo, const double* __restrict__ s, int64_t st, int pt,
+                                                  int k) const
+    {
+        const double c = m[k + 1];
+        const double y = (s[0] * (c - w[k + 1]) + s[1] * (c - e[k])) + (s[st] * (c - m[k]) + s[st + pt] * (c - m[k + 2])) +
+                         (s[2 * st] * (c - w[k]) + s[2 * st + pt + 1] * (c - e[k + 1]));
+        return y + rhs_inner(mc, mo, k);
+    }
     // convection of a row off the walls (difference form: add_convection_v)
     __device__ __forceinline__ double convect(double a, double b, double d, int k) const
     {
@@ -441,7 +456,8 @@ struct PairWindow { // rows i0-1 .. i0+2 of column j, and of its neighbours as f
 // GEN: problems of the batch have a tensor field or advection.
 template <int NT, bool GEN, typename F>
 __device__ __forceinline__ void residual_pair(const LevelProb& P, const FastRows& tab, int i0,
-                                              const double* __restrict__ u, const double* __restrict__ x, bool want_b,
+                                              const double* __restrict__ u, const double* __restrict__ x,
+                                              const double* __restrict__ stiff, int64_t sst, bool want_b,
                                               double (&acc)[2], F&& f)
 {
     const int nx = P.nx, ny = P.ny, pt = P.pitch;
@@ -459,9 +475,24 @@ __device__ __forceinline__ void residual_pair(const LevelProb& P, const FastRows
         double b0 = U.rhs(tab.b[c0][cc], 0), b1 = in1 ? U.rhs(tab.b[c1][cc], 1) : 0.0;
         double r0, r1;
         if (GEN && (P.aniso || P.vel)) {
-            const int64_t at = P.origin + (int64_t)i0 * pt + j;
-            r0 = b0 - X.apply_full(row_coefs<double>(P, i0, j, at), 0);
-            r1 = in1 ? b1 - X.apply_full(row_coefs<double>(P, i0 + 1, j, at + pt), 1) : 0.0;
+            // (one lane's chain at the wall columns, so a short one: the
+            // table's masses with the node's own stiffness)
+            auto row_of = [&](int c, int q) {
+                Row<double> r = tab.a[c][cc];
+                if (P.aniso) {
+                    const double* s = stiff + P.origin + (int64_t)(i0 + q) * pt + j;
+                    r.kw = s[0];
+                    r.ke = s[1];
+                    r.ks = s[sst];
+                    r.kn = s[sst + pt];
+                    r.ksw = s[2 * sst];
+                    r.kne = s[2 * sst + pt + 1];
+                }
+                if (P.vel) add_convection<double>(P, i0 + q, j, P.vel_d, r);
+                return r;
+            };
+            r0 = b0 - X.apply_full(row_of(c0, 0), 0);
+            r1 = in1 ? b1 - X.apply_full(row_of(c1, 1), 1) : 0.0;
         } else {
             r0 = b0 - X.apply(tab.a[c0][cc], 0);
             r1 = in1 ? b1 - X.apply(tab.a[c1][cc], 1) : 0.0;
@@ -483,7 +514,7 @@ __device__ __forceinline__ void residual_pair(const LevelProb& P, const FastRows
 #pragma unroll 1
     for (int e = wave; e < 2; e += NT / 64)
         if ((threadIdx.x & 63) == 0) by_table(e ? nx : 0, e ? 2 : 0);
-    if (inner && !(GEN && P.aniso)) {
+    if (inner) {
         const Row<double>& ra = tab.a[1][1];
         const double mc = ra.mc, mo = ra.mw, kx = ra.kw, ky = ra.ks;
         const double c0 = tab.b[1][1][0], c1 = tab.b[1][1][1], cs = tab.b[1][1][7];
@@ -502,7 +533,15 @@ __device__ __forceinline__ void residual_pair(const LevelProb& P, const FastRows
             U.load(ur, j, row);
             X.load(xr, j, row);
             const double b0 = U.rhs_inner(c0, c1, 0) + cs, b1 = U.rhs_inner(c0, c1, 1) + cs;
-            double r0 = b0 - X.apply_inner(mc, mo, kx, ky, 0), r1 = b1 - X.apply_inner(mc, mo, kx, ky, 1);
+            double r0, r1;
+            if (GEN && P.aniso) {
+                const double* s = stiff + P.origin + (int64_t)i0 * pt + j;
+                r0 = b0 - X.apply_stiff(mc, mo, s, sst, pt, 0);
+                r1 = b1 - X.apply_stiff(mc, mo, s + pt, sst, pt, 1);
+            } else {
+                r0 = b0 - X.apply_inner(mc, mo, kx, ky, 0);
+                r1 = b1 - X.apply_inner(mc, mo, kx, ky, 1);
+            }
             if (vel) {
                 r0 -= X.convect(ca[0], cb[0], cd[0], 0);
                 r1 -= X.convect(ca[1], cb[1], cd[1], 1);
@@ -549,7 +588,8 @@ __global__ __launch_bounds__(NT, GEN ? 4 : fast_waves(sizeof(T), NT, V)) void k_
                                                      const FastProb* __restrict__ fp, const FastRows* __restrict__ rows,
                                                      const FastPlan* __restrict__ plans, const Cx<T>* __restrict__ tab,
                                                      const double* __restrict__ u,
-                                                     const double* __restrict__ x, T* __restrict__ out,
+                                                     const double* __restrict__ x, const double* __restrict__ stiff,
+                                                     int64_t sst, T* __restrict__ out,
                                                      double* __restrict__ partial, CgState* st, int k, int start)
 {
     extern __shared__ char lds_raw[];
@@ -571,7 +611,7 @@ __global__ __launch_bounds__(NT, GEN ? 4 : fast_waves(sizeof(T), NT, V)) void k_
     const int ends = f.ends;
     const T two = (T)2;
     clear_gap<T, NT>(s, pl, N + 1, pl.M - N);
-    residual_pair<NT, GEN>(P, rows[job.prob], i0, u, x, k == 0, acc, [&](int j, double r0, double r1) {
+    residual_pair<NT, GEN>(P, rows[job.prob], i0, u, x, stiff, sst, k == 0, acc, [&](int j, double r0, double r1) {
         Cx<T> v = {(T)r0, (T)r1};
         if (ends == kEndsNN) {
             if (j == 0 || j == N) {

@@ -48,8 +48,8 @@ __global__ __launch_bounds__(256) void k_fast_check(const FastJob* __restrict__ 
                                                     const LevelProb* __restrict__ probs,
                                                     const FastProb* __restrict__ fp, const FastRows* __restrict__ rows,
                                                     const double* __restrict__ u, const double* __restrict__ x,
-                                                    double* __restrict__ partial,
-                                                    const CgState* __restrict__ st)
+                                                    const double* __restrict__ stiff, int64_t sst,
+                                                    double* __restrict__ partial, const CgState* __restrict__ st)
 {
     const int t = swizzled_block();
     if (t >= njobs) return;
@@ -57,7 +57,7 @@ __global__ __launch_bounds__(256) void k_fast_check(const FastJob* __restrict__ 
     const LevelProb& P = probs[job.prob];
     if (st[P.prob].done) return;
     double acc[2] = {0.0, 0.0};
-    residual_pair<256, GEN>(P, rows[job.prob], 2 * job.at, u, x, false, acc, [](int, double, double) {});
+    residual_pair<256, GEN>(P, rows[job.prob], 2 * job.at, u, x, stiff, sst, false, acc, [](int, double, double) {});
     block_pair<256>(acc);
     if (threadIdx.x == 0) partial[2 * (int64_t)(fp[job.prob].pair0 + job.at)] = acc[0];
 }
@@ -315,6 +315,34 @@ __global__ __launch_bounds__(256) void k_fast_commit(const FastJob* __restrict__
     }
 }
 
+// The stiffness weights of the problems with a tensor field.  Formed in the
+// residual from 21 tensor entries a node they made it the largest launch of a
+// solve (800x400, 2 species: 39 us an application, now 20; the wall columns, one
+// lane's chain of such rows, were half of that).
+__global__ __launch_bounds__(256) void k_fast_stiff(const FastJob* __restrict__ jobs, int njobs,
+                                                    const LevelProb* __restrict__ probs, double* __restrict__ stiff,
+                                                    int64_t sst)
+{
+    const int t = swizzled_block();
+    if (t >= njobs) return;
+    const FastJob job = jobs[t];
+    const LevelProb& P = probs[job.prob];
+    if (!P.aniso) return;
+    for (int w = 0; w < 2; ++w) {
+        const int i = 2 * job.at + w;
+        if (i > P.ny) break;
+        for (int j = threadIdx.x; j <= P.nx; j += 256) {
+            const int64_t k = P.origin + (int64_t)i * P.pitch + j;
+            const double* d = P.tens_d + k;
+            Row<double> r;
+            aniso_stiffness<double>(P, i, j, d, d + P.tstride, d + 2 * P.tstride, P.pitch, r);
+            stiff[k] = r.kw;
+            stiff[k + sst] = r.ks;
+            stiff[k + 2 * sst] = r.ksw;
+        }
+    }
+}
+
 // A solve's start: the iterate takes the wall values on held nodes, and zero
 // elsewhere where no solution is kept.
 __global__ __launch_bounds__(256) void k_fast_start(const FastJob* __restrict__ jobs, int njobs,
@@ -491,6 +519,7 @@ void fast_free(eq_batch* b)
     hipFree(F->d_jobs);
     hipFree(F->d_lines);
     hipFree(F->d_modes);
+    hipFree(F->d_stiff);
     hipFree(F->d_tables);
     hipFree(F->d_partial);
     hipFree(F->d_cheb);
@@ -645,8 +674,8 @@ int fast_build(eq_batch* b)
 // ellipse (Manteuffel, Numer. Math. 28, 1977) converges at a known rate, with
 // no inner products: three launches an application, as without them.
 // Per step against the V-cycle CG and BiCGStab: a cell tensor of contrast 2 on
-// 800x400 4.50 -> 1.4 ms (18 applications of 72 us), a flow of s = 0.8 on
-// 901x449 2.54 -> 1.68 (26 of 62 us).
+// 800x400 4.50 -> 0.99 ms (18 applications of 45 us), a flow of s = 0.8 on
+// 901x449 2.54 -> 1.6 (26 of 56 us).
 // Beyond a rate of 1/2 an application the multigrid solvers are taken (a
 // contrast of 9, s = 4/3): there are over 35 applications to a solve.
 int fast_refresh(eq_batch* b)
@@ -707,6 +736,17 @@ int fast_refresh(eq_batch* b)
     const int n = worst > 0.0 ? (int)(todo / std::log(1.0 / worst)) + 1 : 3;
     for (int& r : F->recent[1]) r = std::min(n + most, FastSolver::kGraphs - 1);
     EQ_HIP(hipStreamSynchronize(b->stream));
+    bool aniso = false;
+    for (const LevelProb& P : b->levels[0].probs) aniso = aniso || P.aniso;
+    if (aniso != (F->d_stiff != nullptr)) {
+        fast_drop_graphs(b); // they hold the old address
+        hipFree(F->d_stiff);
+        F->d_stiff = nullptr;
+        F->stiff_stride = b->levels[0].pool;
+        if (aniso && hipMalloc((void**)&F->d_stiff, sizeof(double) * 3 * F->stiff_stride) != hipSuccess)
+            return set_error(EQ_ERR_NOMEM, "stiffness weights");
+        if (aniso) EQ_HIP(hipMemset(F->d_stiff, 0, sizeof(double) * 3 * F->stiff_stride));
+    }
     if (!F->d_cheb && hipMalloc((void**)&F->d_cheb, sizeof(double2) * tab.size()) != hipSuccess)
         return set_error(EQ_ERR_NOMEM, "fast solver tables");
     EQ_HIP(hipMemcpy(F->d_cheb, tab.data(), sizeof(double2) * tab.size(), hipMemcpyHostToDevice));
@@ -752,6 +792,9 @@ static void fast_chunk(eq_batch* b, int k0, int n)
     if (k0 == 0)
         launch(b, EQ_KERNEL_SOLVE_ONCE, 0.0, k_fast_start, dim3(grid8(njobs)), dim3(256), 0, s,
                (const FastJob*)F->d_jobs, njobs, probs, b->xprev, (const CgState*)b->d_state);
+    if (GEN && k0 == 0 && F->d_stiff)
+        launch(b, EQ_KERNEL_SOLVE_ONCE, nodes * 48.0, k_fast_stiff, dim3(grid8(njobs)), dim3(256), 0, s,
+               (const FastJob*)F->d_jobs, njobs, probs, F->d_stiff, F->stiff_stride);
     for (int k = k0; k < k0 + n; ++k) {
         fast_forward<T, GEN>(b, k, k == k0);
         const dim3 lg(grid8(F->nline)), lb(F->line_c * kFastModes);
@@ -769,7 +812,8 @@ static void fast_chunk(eq_batch* b, int k0, int n)
     }
     launch(b, EQ_KERNEL_SOLVE_ONCE, nodes * 16.0, k_fast_check<GEN>, dim3(grid8(njobs)), dim3(256), 0, s,
            (const FastJob*)F->d_jobs, njobs, probs, (const FastProb*)F->d_probs, (const FastRows*)F->d_rows,
-           (const double*)b->u, (const double*)b->xprev, F->d_partial, (const CgState*)b->d_state);
+           (const double*)b->u, (const double*)b->xprev, (const double*)F->d_stiff, F->stiff_stride, F->d_partial,
+           (const CgState*)b->d_state);
     launch(b, EQ_KERNEL_SOLVE_ONCE, nodes * 16.0, k_fast_commit, dim3(grid8(njobs)), dim3(256), 0, s,
            (const FastJob*)F->d_jobs, njobs, probs, (const FastProb*)F->d_probs, b->u, (const double*)b->xprev,
            (const double*)F->d_partial, b->d_state, (const int32_t*)F->d_extra, F->d_met, k0 + n);

@@ -31,7 +31,7 @@ void fast_forward(eq_batch* b, int k, bool start)
                    dim3(grid8(c.njobs)), dim3(NT), c.lds, b->stream, (const FastJob*)F->d_jobs + c.job0, c.njobs,
                    (const LevelProb*)b->levels[0].d_probs, (const FastProb*)F->d_probs, (const FastRows*)F->d_rows,
                    (const FastPlan*)F->d_plans, (const Cx<T>*)F->d_tables, (const double*)b->u, (const double*)b->xprev,
-                   (T*)b->z, F->d_partial, b->d_state, k, start ? 1 : 0);
+                   (const double*)F->d_stiff, F->stiff_stride, (T*)b->z, F->d_partial, b->d_state, k, start ? 1 : 0);
         });
 }
 
