@@ -153,8 +153,11 @@ __global__ __launch_bounds__(256) void k_fast_modes(const LevelProb* __restrict_
 // through four chunks of a wave by shuffles, then once through LDS; walked
 // chunk by chunk by one thread a mode, and with the modes' constants formed in
 // every thread, it took 21.7 us, now 16.6 (32 MB: 6 us); 800x400 14.3 -> 11.1.
-template <typename T, int L>
-__global__ void k_fast_lines(const FastJob* __restrict__ jobs, int njobs, const LevelProb* __restrict__ probs,
+// MANY: more blocks than the chip holds, so waves in flight count: the record
+// is read where it is used (80 registers for 98; 512 uneven traps 865 -> 819
+// us, where the 2000x1000 trap's one round of blocks takes 17.9 for 16.6).
+template <typename T, int L, bool MANY>
+__global__ __launch_bounds__(1024, MANY && sizeof(T) == 4 && L == 16 ? 6 : 4) void k_fast_lines(const FastJob* __restrict__ jobs, int njobs, const LevelProb* __restrict__ probs,
                              const FastProb* __restrict__ fp, const FastMode* __restrict__ modes, T* __restrict__ io,
                              const double* __restrict__ partial, CgState* st, const int32_t* __restrict__ extra,
                              int32_t* met_at, int k)
@@ -178,7 +181,7 @@ __global__ void k_fast_lines(const FastJob* __restrict__ jobs, int njobs, const 
     T v[L];
 #pragma unroll
     for (int l = 0; l < L; ++l) v[l] = (on && l < nl) ? col[(int64_t)l * P.pitch] : (T)0;
-    const FastMode M = modes[f.mode0 + min(q, N)];
+    std::conditional_t<MANY, const FastMode&, const FastMode> M = modes[f.mode0 + min(q, N)];
     if (threadIdx.x == 0) {
         ((int*)(red + 36))[0] = k > 0 ? cs.done : 0;
         ((int*)(red + 36))[1] = k > 0 ? met_at[P.prob] : -1;
@@ -802,12 +805,13 @@ static void fast_chunk(eq_batch* b, int k0, int n)
             launch(b, EQ_KERNEL_BOTTOM, nodes * 2 * sizeof(T), kern, lg, lb, 0, s, (const FastJob*)F->d_lines, F->nline,
                    probs, (const FastProb*)F->d_probs, (const FastMode*)F->d_modes, z, (const double*)F->d_partial, b->d_state, (const int32_t*)F->d_extra, F->d_met, k);
         };
+        const bool many = F->nline > 1024; // four blocks a CU
         if (F->line_rows <= 1024)
-            lines(k_fast_lines<T, 16>);
+            many ? lines(k_fast_lines<T, 16, true>) : lines(k_fast_lines<T, 16, false>);
         else if (F->line_rows <= 2048)
-            lines(k_fast_lines<T, 32>);
+            many ? lines(k_fast_lines<T, 32, true>) : lines(k_fast_lines<T, 32, false>);
         else
-            lines(k_fast_lines<T, 64>);
+            many ? lines(k_fast_lines<T, 64, true>) : lines(k_fast_lines<T, 64, false>);
         fast_backward<T, GEN>(b, k);
     }
     launch(b, EQ_KERNEL_SOLVE_ONCE, nodes * 16.0, k_fast_check<GEN>, dim3(grid8(njobs)), dim3(256), 0, s,

@@ -22,20 +22,19 @@ constexpr size_t kStageWords = 1 << 17;
 
 // Words [k0, k0 + n) of the natural order of rows of w words, between `flat`
 // (its word k0 first) and `rows` (pitch p).  Both sides are walked in order,
-// four words a thread in flight: bound by the memory or the bus.  An uploaded
+// W words a thread in flight: bound by the memory or the bus.  An uploaded
 // field is a new state: the kept solutions are no start for it (restart: the
 // problem's have_prev and have_prev2).
-constexpr int kRowWords = 4;
-template <bool TO_ROWS>
+template <bool TO_ROWS, int W>
 __global__ __launch_bounds__(256) void k_rows(double* __restrict__ flat, double* __restrict__ rows, int64_t k0,
                                               int64_t n, uint32_t w, int64_t p, int32_t* restart)
 {
     if (restart && blockIdx.x == 0 && threadIdx.x < 2) restart[threadIdx.x] = 0;
-    const int64_t first = (int64_t)blockIdx.x * (256 * kRowWords) + threadIdx.x;
-    double v[kRowWords];
-    int64_t at[kRowWords];
+    const int64_t first = (int64_t)blockIdx.x * (256 * W) + threadIdx.x;
+    double v[W];
+    int64_t at[W];
 #pragma unroll
-    for (int q = 0; q < kRowWords; ++q) {
+    for (int q = 0; q < W; ++q) {
         const int64_t k = first + 256 * q, g = k0 + k;
         // (divisions in 32 bits wherever the field allows)
         const int64_t i = (g >> 32) == 0 ? (int64_t)((uint32_t)g / w) : g / (int64_t)w;
@@ -43,7 +42,7 @@ __global__ __launch_bounds__(256) void k_rows(double* __restrict__ flat, double*
         if (k < n) v[q] = TO_ROWS ? flat[k] : rows[at[q]];
     }
 #pragma unroll
-    for (int q = 0; q < kRowWords; ++q)
+    for (int q = 0; q < W; ++q)
         if (first + 256 * q < n) {
             if (TO_ROWS)
                 rows[at[q]] = v[q];
@@ -56,9 +55,13 @@ template <bool TO_ROWS>
 static void launch_rows(eq_batch* b, double* flat, double* rows, int64_t k0, int64_t n, int64_t w, int64_t p,
                         int32_t* restart)
 {
-    constexpr int per = 256 * kRowWords;
-    hipLaunchKernelGGL(k_rows<TO_ROWS>, dim3((unsigned)((n + per - 1) / per)), dim3(256), 0, b->stream, flat, rows, k0, n,
-                       (uint32_t)w, p, restart);
+    // up to one round of threads on the chip (2^19) a word each: there a launch
+    // is latency (0.18 M words 4.0 us with four words a thread, 3.1 with one);
+    // beyond, four in flight
+    const int words = n <= (1 << 19) ? 1 : 4, per = 256 * words;
+    auto kern = words == 1 ? k_rows<TO_ROWS, 1> : k_rows<TO_ROWS, 4>;
+    hipLaunchKernelGGL(kern, dim3((unsigned)((n + per - 1) / per)), dim3(256), 0, b->stream, flat, rows, k0, n, (uint32_t)w,
+                       p, restart);
 }
 
 // Whether the batch's device reads and writes this memory in a kernel; other
