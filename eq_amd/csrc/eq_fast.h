@@ -97,7 +97,9 @@ struct FastSolver {
     FastMode* d_modes = nullptr;
     void* d_tables = nullptr;
     double* d_partial = nullptr; // 2 per row pair
-    // varying coefficients (tensor field, advection): per problem kChebMax
+    bool robin_x = false; // some left or right wall is a Robin wall
+    // beyond the constant operator (tensor field, advection, Robin walls
+    // across x): per problem kChebMax
     // pairs (weight of the correction, weight of the one before); whether
     // every problem's bounds allow the solver; the applications they predict
     double2* d_cheb = nullptr;
@@ -741,7 +743,7 @@ void fast_forward(eq_batch* b, int k, bool start);
 template <typename T, bool GEN>
 void fast_backward(eq_batch* b, int k);
 template <typename T, bool GEN>
-int fast_allow_lds();
+int fast_allow_lds(const FastSolver* F);
 
 inline int grid8(int n) { return 8 * ((n + 7) / 8); }
 

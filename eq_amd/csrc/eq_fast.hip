@@ -486,8 +486,22 @@ static bool make_plan(int N, size_t elem, FastPlan& pl)
     return pl.M <= kFastValuesWide * 1024 && (int64_t)fast_lds_bytes(pl.M, elem) <= kFastLds;
 }
 
+// The Robin walls across x, which P takes as closed: their part of the operator
+// is at most this times P (|u(0)|^2 sqrt((1 + dt gamma) dt D) tanh(W / 2l) is
+// the least energy of P with that end value, l = sqrt(dt D / (1 + dt gamma))).
+static double robin_part(const eq_field_desc& d)
+{
+    const double react = 1.0 + d.dt * d.gamma;
+    double r = 0.0;
+    for (int w : {EQ_WALL_LEFT, EQ_WALL_RIGHT})
+        if (d.wall[w].kind == EQ_BC_ROBIN) r = d.wall[w].r >= 0.0 ? std::max(r, d.wall[w].r) : HUGE_VAL;
+    if (r == 0.0) return 0.0;
+    return d.dt * r / (std::sqrt(react * d.dt * d.D) * std::tanh(0.5 * d.width * std::sqrt(react / (d.dt * d.D))));
+}
+
 // Whether the batch's grids and walls allow the solver: x walls closed or
-// held (their transforms diagonalise the x matrices), rows that fit a block,
+// held (their transforms diagonalise the x matrices) or Robin walls of at most
+// twice the closed operator (over 20 applications there), rows that fit a block,
 // and dt D of at least the square of the larger spacing, where the
 // separable matrix is within a tenth of the operator.
 static bool fast_shape(const eq_batch* b)
@@ -495,8 +509,7 @@ static bool fast_shape(const eq_batch* b)
     const size_t elem = b->mixed ? sizeof(Cx<float>) : sizeof(Cx<double>);
     std::map<int, bool> fits;
     for (const eq_field_desc& d : b->descs) {
-        for (int w : {EQ_WALL_LEFT, EQ_WALL_RIGHT})
-            if (d.wall[w].kind == EQ_BC_ROBIN) return false;
+        if (!(robin_part(d) <= 2.0)) return false;
         if (d.ny + 1 > kFastRowsMax || d.nx > (1 << 15)) return false;
         const double hx = d.width / d.nx, hy = d.height / d.ny, h = std::max(hx, hy);
         if (!(d.dt * d.D >= (1.0 + d.dt * d.gamma) * h * h) || h > 4.0 * std::min(hx, hy)) return false;
@@ -654,8 +667,8 @@ static int fast_build_t(eq_batch* b, FastSolver* F)
     }
     EQ_HIP(hipGetLastError());
     EQ_HIP(hipStreamSynchronize(s)); // the host tables above go out of scope
-    const int rg = fast_allow_lds<T, true>();
-    return rg ? rg : fast_allow_lds<T, false>();
+    const int rg = fast_allow_lds<T, true>(F);
+    return rg ? rg : fast_allow_lds<T, false>(F);
 }
 
 int fast_build(eq_batch* b)
@@ -664,7 +677,10 @@ int fast_build(eq_batch* b)
     if (!fast_shape(b)) return EQ_OK;
     b->fast = new (std::nothrow) FastSolver();
     if (!b->fast) return set_error(EQ_ERR_NOMEM, "host allocation");
-    return b->mixed ? fast_build_t<float>(b, b->fast) : fast_build_t<double>(b, b->fast);
+    for (const eq_field_desc& d : b->descs)
+        for (int w : {EQ_WALL_LEFT, EQ_WALL_RIGHT}) b->fast->robin_x = b->fast->robin_x || d.wall[w].kind == EQ_BC_ROBIN;
+    const int rc = b->mixed ? fast_build_t<float>(b, b->fast) : fast_build_t<double>(b, b->fast);
+    return rc || !b->fast->robin_x ? rc : fast_refresh(b);
 }
 
 // Varying coefficients: the spectrum of P^-1 A, with P the constant operator
@@ -679,6 +695,8 @@ int fast_build(eq_batch* b)
 // Per step against the V-cycle CG and BiCGStab: a cell tensor of contrast 2 on
 // 800x400 4.50 -> 0.99 ms (18 applications of 45 us), a flow of s = 0.8 on
 // 901x449 2.54 -> 1.6 (26 of 56 us).
+// Robin walls at a rate of 1.5 on the left and right, 1057x810 in FP64: 2.74 ->
+// 1.41 (six applications).
 // Beyond a rate of 1/2 an application the multigrid solvers are taken (a
 // contrast of 9, s = 4/3): there are over 35 applications to a solve.
 int fast_refresh(eq_batch* b)
@@ -693,8 +711,9 @@ int fast_refresh(eq_batch* b)
     int most = 0;
     for (int p = 0; p < b->nprob; ++p) {
         const LevelProb& P = b->levels[0].probs[p];
-        if (!P.aniso && !P.vel) continue;
         const eq_field_desc& D = b->descs[p];
+        const double robin = robin_part(D);
+        if (!P.aniso && !P.vel && robin == 0.0) continue;
         const double h = std::max(P.hx, P.hy), react = 1.0 + D.dt * D.gamma;
         const double off = react * h * h / (6.0 * D.dt * D.D); // the mass couplings that P leaves out
         double lo = 1.0, hi = 1.0, s = 0.0;
@@ -711,6 +730,7 @@ int fast_refresh(eq_batch* b)
             for (double v : b->vel_host[p][0]) w = std::max(w, std::isfinite(v) ? std::fabs(v) : HUGE_VAL);
             s = 0.5 * w * std::sqrt(D.dt / (react * D.D));
         }
+        hi += robin;
         const double d = 0.5 * (lo + hi), a = 0.5 * (hi - lo) + off, c2 = a * a - s * s;
         const double rate = (a + s) / (d + std::sqrt(d * d - c2));
         if (!(lo > 0.0) || !(rate <= 0.5) || (P.vel && !bicg)) {
@@ -722,8 +742,8 @@ int fast_refresh(eq_batch* b)
         // largest eigenvalue) that the error does not share, so a tighter
         // tolerance may be out of reach: a fixed number of applications takes
         // the error down to the multigrid solvers' (another factor of 100,
-        // 1000 with flow; 3.5e-12 -> 5e-14 and 4.5e-11 -> 2e-13 of the field).
-        extra[p] = rate > 0.0 ? (int)std::ceil(std::log(P.vel ? 1000.0 : 100.0) / std::log(1.0 / rate)) : 0;
+        // 1000 with flow, 10 for Robin walls alone; 3.5e-12 -> 5e-14 and 4.5e-11 -> 2e-13 of the field).
+        extra[p] = rate > 0.0 ? (int)std::ceil(std::log(P.vel ? 1000.0 : P.aniso ? 100.0 : 10.0) / std::log(1.0 / rate)) : 0;
         most = std::max(most, extra[p]);
         double2* w = tab.data() + (size_t)p * kChebMax;
         double al = 1.0 / d;
@@ -766,10 +786,11 @@ bool fast_applies(const eq_batch* b)
     eq_solver_desc d;
     eq_solver_default(&d);
     const eq_solver_desc& S = b->solver;
-    if (b->any_tensor && (!b->fast->general_ok || S.max_iter < kChebMax)) return false;
+    const bool varying = b->any_tensor || b->fast->robin_x;
+    if (varying && (!b->fast->general_ok || S.max_iter < kChebMax)) return false;
     // (an application is a refinement step, and those are few)
     if (S.kind == EQ_SOLVER_IR_GMG_CG &&
-        (b->any_tensor || S.ir_max_outer != d.ir_max_outer || S.ir_inner_rtol != d.ir_inner_rtol))
+        (varying || S.ir_max_outer != d.ir_max_outer || S.ir_inner_rtol != d.ir_inner_rtol))
         return false;
     return S.mg_pre == d.mg_pre && S.mg_post == d.mg_post && S.mg_omega == d.mg_omega && S.mg_omega2 == d.mg_omega2 &&
            S.mg_coarse_max_nodes == d.mg_coarse_max_nodes && S.mg_max_levels == d.mg_max_levels &&
@@ -835,7 +856,7 @@ static int fast_solve_t(eq_batch* b, bool profiling, bool* handled)
     hipStream_t s = b->stream;
     *handled = true;
     const bool graphs = S.use_graphs && !profiling;
-    const int gen = b->any_tensor ? 1 : 0;
+    const int gen = b->any_tensor || F->robin_x ? 1 : 0;
     auto applications = [&](int k0, int n) {
         if (gen)
             fast_chunk<T, true>(b, k0, n);

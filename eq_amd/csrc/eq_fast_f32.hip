@@ -2,7 +2,7 @@
 #include "eq_fast_launch.h"
 
 namespace eqk {
-template int fast_allow_lds<float, false>();
+template int fast_allow_lds<float, false>(const FastSolver*);
 template void fast_forward<float, false>(eq_batch*, int, bool);
 template void fast_backward<float, false>(eq_batch*, int);
 } // namespace eqk

@@ -2,7 +2,7 @@
 #include "eq_fast_launch.h"
 
 namespace eqk {
-template int fast_allow_lds<double, false>();
+template int fast_allow_lds<double, false>(const FastSolver*);
 template void fast_forward<double, false>(eq_batch*, int, bool);
 template void fast_backward<double, false>(eq_batch*, int);
 } // namespace eqk

@@ -6,13 +6,14 @@
 
 namespace eqk {
 
+// (a launch within 64 KiB needs no leave)
 template <typename T, bool GEN>
-int fast_allow_lds()
+int fast_allow_lds(const FastSolver* F)
 {
     int rc = EQ_OK;
-    for (int nt = 64; nt <= 2048; nt *= 2)
-        by_threads(nt, [&](auto c) {
-            constexpr int NT = std::min(1024, decltype(c)::value), V = decltype(c)::value / NT * kFastValues;
+    for (const FastClass& c : F->classes)
+        if (c.lds > 64 * 1024) by_threads(c.threads, [&](auto t) {
+            constexpr int NT = std::min(1024, decltype(t)::value), V = decltype(t)::value / NT * kFastValues;
             for (const void* k : {(const void*)k_fast_forward<T, NT, V, GEN>, (const void*)k_fast_backward<T, NT, V, GEN>})
                 if (hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kFastLds) != hipSuccess)
                     rc = set_error(EQ_ERR_HIP, "hipFuncSetAttribute");

@@ -96,3 +96,30 @@ def test_advection_still_needs_a_bicgstab_solver(eqf):
         with pytest.raises(eqf.EqError) as e:
             fb.step()
         assert e.value.code == 1
+
+
+@pytest.mark.parametrize("kind", ["GMG_CG", "MIXED_GMG_CG", "MIXED_GMG_BICGSTAB"])
+@pytest.mark.parametrize("left,right", [(1.5, 1.5), (0.0, 1.5), (None, 30.0), (50.0, None), (60.0, 400.0)])
+@pytest.mark.parametrize("fd", [False, True])
+def test_robin_walls_across_x(eqf, oracle, kind, left, right, fd):
+    """Rates from none to past the bound (twice the closed operator), one or
+    both walls, the other held; a step of every kind with them."""
+    w = {oracle.TOP: (oracle.DIRICHLET, 0.25, 0.0, 0.0)}
+    for wall, r in ((oracle.LEFT, left), (oracle.RIGHT, right)):
+        w[wall] = (oracle.DIRICHLET, 0.5, 0.0, 0.0) if r is None else (oracle.ROBIN, 0.0, r, 0.2)
+    rng = np.random.default_rng(11)
+    descs, probs, u = [], [], []
+    for k, (nx, ny) in enumerate(SHAPES):
+        # (the finite-difference oracle has no reaction and no source)
+        args = (nx, ny, nx * H, ny * H, DT, 60.0 + 20 * k) + ((0.0, 0.0) if fd else (0.01, 0.05))
+        descs.append(eqf.field_desc(*args, w, scheme=eqf.SCHEME_FD if fd else eqf.SCHEME_P1))
+        probs.append(oracle.problem(*args, walls=w))
+        u.append(rng.random((nx + 1) * (ny + 1)))
+    with eqf.FieldBatch(descs, solver=eqf.solver_desc(getattr(eqf, kind))) as fb:
+        for k in range(len(descs)):
+            fb.upload(k, u[k])
+        for step in range(2):
+            assert fb.step().nconverged == len(descs)
+            for k, p in enumerate(probs):
+                u[k] = oracle.fd_step(p, u[k]) if fd else oracle.step(p, u[k], "lu")[0]
+                assert _rel(fb.download(k), u[k]) <= 1e-9, (step, k)
