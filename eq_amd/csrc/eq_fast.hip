@@ -1,4 +1,5 @@
-// eq_fast.hip -- the constant-coefficient field step by a fast direct solver.
+// eq_fast.hip -- the field step by a fast direct solver (varying coefficients
+// and Robin walls across x: as the operator of a Chebyshev iteration, fast_refresh).
 //
 // With constant coefficients the P1 operator on the uniform "right"-diagonal
 // mesh is separable but for one term: the stiffness is Kx (x) Ly + Lx (x) Ky
@@ -16,9 +17,9 @@
 // The finite-difference scheme is separable exactly.
 //
 // Measured per time step, couple + solve + fields out, against the V-cycle
-// CG: 2000x1000, 2 species 2.58 -> 0.40 ms (FP64 3.04 -> 0.46), 1237x611 (a
-// chirp length) 2.02 -> 0.34, 12 uneven traps 3.32 -> 1.02, 512 uneven traps
-// 69.4 -> 28.0; errors against a 64-bit solve 4e-15 to 6e-13.
+// CG: 2000x1000, 2 species 2.57 -> 0.39 ms (FP64 3.04 -> 0.44), 1237x611 (a
+// chirp length) 2.01 -> 0.33, 12 uneven traps 3.32 -> 1.03, 512 uneven traps
+// 69.8 -> 28.2; errors against a 64-bit solve 4e-15 to 6e-13.
 //
 // What bounds the transforms: vector issue and latency, not bandwidth
 // (2000x1000: forward 34 us, backward 28, where the bytes take 18 and 14).
@@ -486,6 +487,11 @@ static bool make_plan(int N, size_t elem, FastPlan& pl)
     return pl.M <= kFastValuesWide * 1024 && (int64_t)fast_lds_bytes(pl.M, elem) <= kFastLds;
 }
 
+static bool robin_x(const eq_field_desc& d)
+{
+    return d.wall[EQ_WALL_LEFT].kind == EQ_BC_ROBIN || d.wall[EQ_WALL_RIGHT].kind == EQ_BC_ROBIN;
+}
+
 // The Robin walls across x, which P takes as closed: their part of the operator
 // is at most this times P (|u(0)|^2 sqrt((1 + dt gamma) dt D) tanh(W / 2l) is
 // the least energy of P with that end value, l = sqrt(dt D / (1 + dt gamma))).
@@ -501,7 +507,9 @@ static double robin_part(const eq_field_desc& d)
 
 // Whether the batch's grids and walls allow the solver: x walls closed or
 // held (their transforms diagonalise the x matrices) or Robin walls of at most
-// twice the closed operator (over 20 applications there), rows that fit a block,
+// twice the closed operator (over 20 applications there; in every problem of
+// the batch or none: mixed batches keep the multigrid solvers, whose iteration
+// counts on them are relied on), rows that fit a block,
 // and dt D of at least the square of the larger spacing, where the
 // separable matrix is within a tenth of the operator.
 static bool fast_shape(const eq_batch* b)
@@ -509,7 +517,7 @@ static bool fast_shape(const eq_batch* b)
     const size_t elem = b->mixed ? sizeof(Cx<float>) : sizeof(Cx<double>);
     std::map<int, bool> fits;
     for (const eq_field_desc& d : b->descs) {
-        if (!(robin_part(d) <= 2.0)) return false;
+        if (!(robin_part(d) <= 2.0) || robin_x(d) != robin_x(b->descs[0])) return false;
         if (d.ny + 1 > kFastRowsMax || d.nx > (1 << 15)) return false;
         const double hx = d.width / d.nx, hy = d.height / d.ny, h = std::max(hx, hy);
         if (!(d.dt * d.D >= (1.0 + d.dt * d.gamma) * h * h) || h > 4.0 * std::min(hx, hy)) return false;
@@ -677,8 +685,7 @@ int fast_build(eq_batch* b)
     if (!fast_shape(b)) return EQ_OK;
     b->fast = new (std::nothrow) FastSolver();
     if (!b->fast) return set_error(EQ_ERR_NOMEM, "host allocation");
-    for (const eq_field_desc& d : b->descs)
-        for (int w : {EQ_WALL_LEFT, EQ_WALL_RIGHT}) b->fast->robin_x = b->fast->robin_x || d.wall[w].kind == EQ_BC_ROBIN;
+    b->fast->robin_x = robin_x(b->descs[0]); // (all of them)
     const int rc = b->mixed ? fast_build_t<float>(b, b->fast) : fast_build_t<double>(b, b->fast);
     return rc || !b->fast->robin_x ? rc : fast_refresh(b);
 }

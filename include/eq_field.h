@@ -102,12 +102,14 @@ typedef enum {
                                    correction solved by CG in FP32 (FP32 vectors and
                                    stencil, FP32 V-cycle) to ir_inner_rtol          */
 } eq_solver_kind;
-/* GMG_CG and MIXED_GMG_CG with the cycle options (mg_*, tile*, extrapolate) at
- * their defaults: a batch of constant coefficients whose left and right walls
- * are not Robin is solved by a fast direct solver in the kind's precision
+/* With the cycle options (mg_*, tile*, extrapolate, ir_*) at their defaults the
+ * multigrid kinds are solved by a fast direct solver in the kind's precision
  * (same tolerance on the same FP64 residual), iterations counting its
- * applications; a batch with a tensor field, and a caller that sets a cycle,
- * get that multigrid cycle. */
+ * applications: constant coefficients directly, tensor fields of a contrast up
+ * to 9, velocities up to (8/3) sqrt(D / dt) (BiCGStab kinds) and Robin walls on
+ * the left and right of every problem by a Chebyshev iteration on it (not
+ * IR_GMG_CG; max_iter at least 64).  Other batches, and a caller that sets a
+ * cycle, get that multigrid cycle. */
 
 typedef struct {
     int32_t kind;                /* eq_solver_kind                                  */
