@@ -377,6 +377,22 @@ __device__ __forceinline__ void clear_gap(Cx<T>* s, const FastPlan& pl, int a, i
     for (int k = a + (int)threadIdx.x; k <= b; k += NT) s[k] = {(T)0, (T)0};
 }
 
+// The residual's scale.  Single precision holds the residual of a solve, from
+// about the right-hand side to 1e-12 of it, only within its own range of
+// exponents, so it is transformed times 2^-e (exact), e the exponent of the
+// problem's first residual and right-hand side, and what comes back is added
+// times 2^e.  The first launch of a solve takes the e of the solve before, and
+// finds its own norms: within kFastScaleOff of them e stays (the 250 exponents
+// leave room), else that launch's transform is dropped, the next one starts
+// with the new e.  The results are the same bits whatever e is.
+constexpr int kFastScaleOff = 32;
+
+template <typename T>
+__device__ __forceinline__ double scale_down(const CgState& cs, int k)
+{
+    return sizeof(T) == 4 ? ldexp(1.0, -(k == 0 ? cs.fast_e0 : cs.fast_e)) : 1.0;
+}
+
 // waves per SIMD the transform kernels are compiled for
 constexpr int fast_waves(size_t elem, int NT, int V) { return V > kFastValues ? 4 : elem == 4 ? 8 : 4; }
 
@@ -612,9 +628,10 @@ __global__ __launch_bounds__(NT, GEN ? 4 : fast_waves(sizeof(T), NT, V)) void k_
     double acc[2] = {0.0, 0.0};
     const int ends = f.ends;
     const T two = (T)2;
+    const double down = scale_down<T>(cs, k);
     clear_gap<T, NT>(s, pl, N + 1, pl.M - N);
     residual_pair<NT, GEN>(P, rows[job.prob], i0, u, x, stiff, sst, k == 0, acc, [&](int j, double r0, double r1) {
-        Cx<T> v = {(T)r0, (T)r1};
+        Cx<T> v = {(T)(r0 * down), (T)(r1 * down)};
         if (ends == kEndsNN) {
             if (j == 0 || j == N) {
                 put_at(s, pl, tab, j, Cx<T>{two * v.x, two * v.y});
@@ -652,8 +669,9 @@ __global__ __launch_bounds__(NT, GEN ? 4 : fast_waves(sizeof(T), NT, V)) void k_
     });
 }
 
-// Transform back along x and x += z, two rows a block.  GEN: application k of
-// the Chebyshev iteration, d <- alpha_k z + beta_k d, x += d.
+// Transform back along x and x += z, two rows a block.  GEN: one application of
+// the Chebyshev iteration, d <- alpha z + beta d, x += d (d in z's scale, which
+// a solve keeps).
 template <typename T, int NT, int V, bool GEN>
 __global__ __launch_bounds__(NT, fast_waves(sizeof(T), NT, V)) void k_fast_backward(const FastJob* __restrict__ jobs, int njobs,
                                                       const LevelProb* __restrict__ probs,
@@ -671,6 +689,9 @@ __global__ __launch_bounds__(NT, fast_waves(sizeof(T), NT, V)) void k_fast_backw
     const LevelProb& P = probs[job.prob];
     const CgState& cs = st[P.prob];
     if (cs.done) return;
+    const int app = k - cs.fast_void; // the application of this solve
+    if (app < 0) return;
+    const double up = sizeof(T) == 4 ? ldexp(1.0, cs.fast_e) : 1.0;
     const FastProb f = fp[job.prob];
     const FastPlan& pl = plans[f.plan];
     const int N = pl.N, i0 = 2 * job.at, ends = f.ends;
@@ -698,7 +719,7 @@ __global__ __launch_bounds__(NT, fast_waves(sizeof(T), NT, V)) void k_fast_backw
     [[maybe_unused]] T* __restrict__ dr = GEN ? d + P.origin + (int64_t)i0 * P.pitch : nullptr;
     [[maybe_unused]] T al = (T)1, be = (T)0;
     if constexpr (GEN) {
-        const double2 w = cheb[(int64_t)job.prob * kChebMax + min(k, kChebMax - 1)];
+        const double2 w = cheb[(int64_t)job.prob * kChebMax + min(app, kChebMax - 1)];
         al = (T)w.x;
         be = (T)w.y;
     }
@@ -711,13 +732,13 @@ __global__ __launch_bounds__(NT, fast_waves(sizeof(T), NT, V)) void k_fast_backw
             v = mul(v, tab[pl.quart + jj]);
         if (j < jlo || j > jhi) return;
         if constexpr (GEN) {
-            if (k > 0) v = Cx<T>{al * v.x + be * dr[j], al * v.y + (second ? be * dr[j + pitch] : (T)0)};
+            if (app > 0) v = Cx<T>{al * v.x + be * dr[j], al * v.y + (second ? be * dr[j + pitch] : (T)0)};
             else v = Cx<T>{al * v.x, al * v.y};
             dr[j] = v.x;
             if (second) dr[j + pitch] = v.y;
         }
-        if (!held0 && !top0) xr[j] += (double)v.x;
-        if (second && !held1) xr[j + pitch] += (double)v.y;
+        if (!held0 && !top0) xr[j] += up * (double)v.x;
+        if (second && !held1) xr[j + pitch] += up * (double)v.y;
     });
 }
 

@@ -191,21 +191,37 @@ __global__ __launch_bounds__(1024, MANY && sizeof(T) == 4 && L == 16 ? 6 : 4) vo
     sum_pairs(partial + 2 * (int64_t)f.pair0, f.npairs, red, rr, bb);
     if (((int*)(red + 36))[0]) return;
     if (k > 0) bb = cs.bb;
+    // the first launch settles the scale (fast_e0 is not written here, so every block finds the same)
+    int e = 0, drop = 0;
+    if (sizeof(T) == 4 && k == 0) {
+        const double msq = (rr + bb) / ((double)rows * (double)(N + 1));
+        e = cs.fast_e0;
+        if (msq > 0.0 && msq < HUGE_VAL) {
+            const int own = ilogb(msq) / 2;
+            drop = own > e + kFastScaleOff || own < e - kFastScaleOff;
+            if (drop) e = own;
+        }
+    }
+    const int app = k == 0 ? 0 : max(0, k - cs.fast_void); // applications done
     // (a block that already reads the first block's entry takes the same way)
     const bool conv = rr <= cs.tol2 * bb;
     int first = ((int*)(red + 36))[1];
-    if (conv && first < 0) first = k;
-    const bool stop = (conv && k >= first + extra[job.prob]) || k >= cs.max_iter;
+    if (conv && first < 0) first = app;
+    const bool stop = (conv && app >= first + extra[job.prob]) || app >= cs.max_iter;
     if (job.at == 0 && threadIdx.x == 0) {
-        if (k == 0) cs.bb = bb;
+        if (k == 0) {
+            cs.bb = bb;
+            cs.fast_void = drop;
+            cs.fast_e = e;
+        }
         met_at[P.prob] = first;
         cs.done = stop ? 1 : 0;
         if (stop) {
-            cs.fast_iter = k;
+            cs.fast_iter = app;
             cs.rr_true = rr;
         }
     }
-    if (stop) return;
+    if (stop || drop) return;
     const double rho = M.rho;
     // chunk ends from zero carries: F at the chunk's last row, G before its first
     double F = 0.0, G = 0.0;
@@ -295,11 +311,13 @@ __global__ __launch_bounds__(256) void k_fast_commit(const FastJob* __restrict__
     if (was == 2) return;
     // (a block that already reads the first block's `done` takes the same way)
     const bool conv = rr <= cs.tol2 * cs.bb;
-    const int first = conv && met < 0 ? k : met;
-    const bool over = was || (conv && k >= first + extra[job.prob]) || k >= cs.max_iter;
+    const int app = k - cs.fast_void;
+    const int first = conv && met < 0 ? app : met;
+    const bool over = was || (conv && app >= first + extra[job.prob]) || app >= cs.max_iter;
     if (job.at == 0 && threadIdx.x == 0) {
+        cs.fast_e0 = cs.fast_e;
         if (!was) {
-            cs.fast_iter = k;
+            cs.fast_iter = app;
             met_at[P.prob] = first;
             cs.rr_true = rr;
         }

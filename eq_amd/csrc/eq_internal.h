@@ -65,8 +65,10 @@ struct CgState {
     int32_t extrap;         // extrapolation allowed (solver setting)
     // BiCGStab: rho = (r^, r), omega, and the pieces of omega
     double rho, omega, ts, tt;
-    int32_t fast_iter;      // fast direct solver: applications when the problem stopped
-    int32_t pad_;
+    // fast direct solver: applications when the problem stopped; launches of
+    // this solve that only set the scale (0 or 1); the scale's exponent at a
+    // solve's start and from its second launch on
+    int32_t fast_iter, fast_void, fast_e0, fast_e;
 };
 
 struct FastSolver; // eq_fast.hip
