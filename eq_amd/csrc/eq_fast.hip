@@ -207,7 +207,7 @@ __global__ __launch_bounds__(1024, MANY && sizeof(T) == 4 && L == 16 ? 6 : 4) vo
     const bool conv = rr <= cs.tol2 * bb;
     int first = ((int*)(red + 36))[1];
     if (conv && first < 0) first = app;
-    const bool stop = (conv && app >= first + extra[job.prob]) || app >= cs.max_iter;
+    const bool stop = conv && app >= first + extra[job.prob];
     if (job.at == 0 && threadIdx.x == 0) {
         if (k == 0) {
             cs.bb = bb;
@@ -286,8 +286,8 @@ __global__ __launch_bounds__(1024, MANY && sizeof(T) == 4 && L == 16 ? 6 : 4) vo
 }
 
 // The chunk's end: every block takes its problem's residual norm, and where
-// the solve is over (converged or out of iterations) the iterate becomes the
-// field.  The first block of a problem keeps its state.
+// the solve has converged the iterate becomes the field (any other field stays
+// as the step found it).  The first block of a problem keeps its state.
 __global__ __launch_bounds__(256) void k_fast_commit(const FastJob* __restrict__ jobs, int njobs,
                                                      const LevelProb* __restrict__ probs,
                                                      const FastProb* __restrict__ fp, double* __restrict__ u,
@@ -313,7 +313,7 @@ __global__ __launch_bounds__(256) void k_fast_commit(const FastJob* __restrict__
     const bool conv = rr <= cs.tol2 * cs.bb;
     const int app = k - cs.fast_void;
     const int first = conv && met < 0 ? app : met;
-    const bool over = was || (conv && app >= first + extra[job.prob]) || app >= cs.max_iter;
+    const bool over = was || (conv && app >= first + extra[job.prob]);
     if (job.at == 0 && threadIdx.x == 0) {
         cs.fast_e0 = cs.fast_e;
         if (!was) {
@@ -869,10 +869,10 @@ static void fast_chunk(eq_batch* b, int k0, int n)
            (const double*)F->d_partial, b->d_state, (const int32_t*)F->d_extra, F->d_met, k0 + n);
 }
 
-// One step's solve.  handled = false: the residual did not reach the tolerance
-// in kFastGiveUp applications and iterations are left; the multigrid solver
-// then continues from the kept iterate (the problems already solved are
-// listed in `solved`, their fields final).
+// One step's solve.  handled = false: some residual did not reach the tolerance
+// in the applications given to it, at most the kind's iteration limit; those
+// problems (h_state: not done) still hold the step's fields, for the multigrid
+// solver to take, and the others their solutions.
 template <typename T>
 static int fast_solve_t(eq_batch* b, bool profiling, bool* handled)
 {
@@ -890,7 +890,9 @@ static int fast_solve_t(eq_batch* b, bool profiling, bool* handled)
     };
     int* recent = F->recent[gen];
     int chunk = *std::max_element(recent, recent + 4);
-    chunk = std::max(1, std::min({chunk, S.max_iter, FastSolver::kGraphs - 1}));
+    const int limit = S.kind == EQ_SOLVER_IR_GMG_CG ? S.ir_max_outer : S.max_iter;
+    const int give_up = std::min(gen ? kChebMax : kFastGiveUp, limit);
+    chunk = std::max(1, std::min({chunk, give_up, FastSolver::kGraphs - 1}));
     for (int k0 = 0;;) {
         if (k0 == 0 && graphs) {
             hipGraphExec_t& ge = F->graph[chunk];
@@ -921,11 +923,11 @@ static int fast_solve_t(eq_batch* b, bool profiling, bool* handled)
         bool all = true;
         for (int p = 0; p < b->nprob; ++p) all = all && b->h_state[p].done;
         if (all) break;
-        if (k0 >= (gen ? kChebMax : kFastGiveUp) && k0 < S.max_iter) {
+        if (k0 >= give_up) {
             *handled = false;
             return EQ_OK;
         }
-        chunk = std::max(1, std::min(2, S.max_iter - k0));
+        chunk = std::min(2, give_up - k0);
     }
     int most = 1;
     for (int p = 0; p < b->nprob; ++p) most = std::max(most, b->h_state[p].iter);
