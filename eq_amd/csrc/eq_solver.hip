@@ -4444,6 +4444,11 @@ static int run_solve(eq_batch* b, eq_step_stats* stats)
     prof_collect(b);
     if (handled) return report_solve(b, stats, t0);
     const std::vector<CgState> solved(b->h_state, b->h_state + b->nprob);
+    // the iterates that did not get there are no start (they may have stalled
+    // or diverged): those problems start from their fields
+    for (int p = 0; p < b->nprob; ++p)
+        if (!solved[p].done) b->h_state[p].have_prev = b->h_state[p].have_prev2 = 0;
+    EQ_HIP(hipMemcpyAsync(b->d_state, b->h_state, sizeof(CgState) * b->nprob, hipMemcpyHostToDevice, b->stream));
     const size_t bytes = sizeof(double) * b->levels[0].pool;
     double* kept = nullptr;
     if (hipMalloc((void**)&kept, bytes) != hipSuccess) return set_error(EQ_ERR_NOMEM, "solved fields");

@@ -31,3 +31,38 @@ def test_iteration_limits_that_the_cycles_meet(eqf, oracle, solver, spare):
         fb.upload(0, u)
         assert fb.step().nconverged == 1, need
         assert _rel(fb.download(0), ref) <= 1e-9
+
+
+@pytest.mark.parametrize("solver", ["GMG_CG", "MIXED_GMG_CG"])
+def test_a_tensor_set_over_the_cells_tensor(eqf, oracle, solver):
+    """A tensor field set on a problem whose cells drive its tensor, then rods
+    that write it again: the operator's eigenvalues are the cells', not the set
+    field's.  Each step, from a kept solution and after a step that went wrong
+    or right, is the oracle's."""
+    import torch
+    nx, ny, npm = 96, 48, 8.0
+    walls = {oracle.TOP: (oracle.DIRICHLET, 0.0, 0.0, 0.0)}
+    args = (nx, ny, nx / npm, ny / npm, DT, 60.0, 0.01, 0.0)
+    rng = np.random.default_rng(3)
+    n, nc = (nx + 1) * (ny + 1), 60
+    cells = np.column_stack([rng.uniform(0, nx / npm, nc), rng.uniform(0, ny / npm, nc), rng.uniform(0, 3, nc),
+                             rng.uniform(2, 4, nc), np.ones(nc)])
+    u = rng.random(n)
+    cells_d = torch.from_numpy(cells).cuda()
+    q_d = torch.from_numpy(rng.random((nc, 1)) * 0.1).cuda()
+    samp = torch.zeros((nc, 1), dtype=torch.float64, device="cuda")
+    cnt = torch.zeros(nc, dtype=torch.int32, device="cuda")
+    torch.cuda.synchronize()
+    p = oracle.problem(*args, walls=walls)
+    with eqf.FieldBatch([eqf.field_desc(*args, walls)], solver=eqf.solver_desc(getattr(eqf, solver))) as fb:
+        fb.upload(0, u)
+        fb.cell_tensor(0, 7.0, 1.0)
+        for step in range(4):
+            if step == 2:
+                fb.set_tensor(0, np.ones(n), np.ones(n), np.zeros(n))
+            fb.couple_dev(0, cells_d.data_ptr(), nc, npm, q_d.data_ptr(), samp.data_ptr(), cnt.data_ptr(),
+                          eqf.SAMPLE | eqf.DEPOSIT | eqf.TENSOR)
+            before, t = fb.download(0), fb.tensor_values(0)
+            assert fb.step().nconverged == 1, step
+            ref, _ = oracle.step(p, before, "lu", D11=t[0], D22=t[1], D12=t[2])
+            assert _rel(fb.download(0), ref) <= 1e-9, step
