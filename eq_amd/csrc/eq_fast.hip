@@ -749,6 +749,10 @@ int fast_refresh(eq_batch* b)
             }
             lo = std::min(lo, b->tens_bounds[p][0]);
             hi = std::max(hi, b->tens_bounds[p][1]);
+            if (P.celltens) { // a coupling may write over a field that was set
+                lo = std::min(lo, b->cell_bounds[p][0]);
+                hi = std::max(hi, b->cell_bounds[p][1]);
+            }
         }
         if (P.vel) {
             double w = 0.0;

@@ -296,6 +296,7 @@ struct eq_batch {
     float** d_tens32 = nullptr;
     std::vector<int32_t> cell_tensor_traps;
     std::vector<std::array<double, 2>> tens_bounds; // per problem: least and largest eigenvalue of its tensor field
+    std::vector<std::array<double, 2>> cell_bounds; // the same of what the cells write (celltens problems)
     bool coarse_tensors_stale = false; // the finest level's tensors have still to be carried to the coarse levels
     std::vector<eqk::InvJob> inv_jobs;
     eqk::InvJob* d_inv_jobs = nullptr;

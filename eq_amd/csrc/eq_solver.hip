@@ -5011,7 +5011,8 @@ int eq_batch_cell_tensor(eq_batch* b, int32_t trap, double Dx, double Dy, int32_
         std::vector<double> one(n, 1.0), zero(n, 0.0);
         for (int p = p0; p < p0 + ns; ++p) {
             if ((rc = set_tensor_checked(b, p, one.data(), one.data(), zero.data(), n))) return rc;
-            b->tens_bounds[p] = {std::min({1.0, Dx, Dy}), std::max({1.0, Dx, Dy})};
+            b->cell_bounds.resize(b->nprob, {1.0, 1.0});
+            b->cell_bounds[p] = {std::min({1.0, Dx, Dy}), std::max({1.0, Dx, Dy})};
         }
     } else {
         for (int p = p0; p < p0 + ns; ++p)
