@@ -728,10 +728,10 @@ int fast_refresh(eq_batch* b)
 {
     FastSolver* F = b->fast;
     if (!F) return EQ_OK;
+    F->general_ok = false; // until everything below is in place
     const bool bicg = b->solver.kind == EQ_SOLVER_GMG_BICGSTAB || b->solver.kind == EQ_SOLVER_MIXED_GMG_BICGSTAB;
     std::vector<double2> tab((size_t)b->nprob * kChebMax, make_double2(1.0, 0.0));
     std::vector<int32_t> extra(b->nprob, 0);
-    F->general_ok = true;
     double worst = 0.0;
     int most = 0;
     for (int p = 0; p < b->nprob; ++p) {
@@ -743,10 +743,7 @@ int fast_refresh(eq_batch* b)
         const double off = react * h * h / (6.0 * D.dt * D.D); // the mass couplings that P leaves out
         double lo = 1.0, hi = 1.0, s = 0.0;
         if (P.aniso) {
-            if ((int)b->tens_bounds.size() <= p) {
-                F->general_ok = false;
-                break;
-            }
+            if ((int)b->tens_bounds.size() <= p) return EQ_OK;
             lo = std::min(lo, b->tens_bounds[p][0]);
             hi = std::max(hi, b->tens_bounds[p][1]);
             if (P.celltens) { // a coupling may write over a field that was set
@@ -762,10 +759,7 @@ int fast_refresh(eq_batch* b)
         hi += robin;
         const double d = 0.5 * (lo + hi), a = 0.5 * (hi - lo) + off, c2 = a * a - s * s;
         const double rate = (a + s) / (d + std::sqrt(d * d - c2));
-        if (!(lo > 0.0) || !(rate <= 0.5) || (P.vel && !bicg)) {
-            F->general_ok = false;
-            break;
-        }
+        if (!(lo > 0.0) || !(rate <= 0.5) || (P.vel && !bicg)) return EQ_OK;
         worst = std::max(worst, rate);
         // The residual has a floor of rounding (the iterate's own, times the
         // largest eigenvalue) that the error does not share, so a tighter
@@ -782,7 +776,6 @@ int fast_refresh(eq_batch* b)
             w[k] = make_double2(al, d * al - 1.0);
         }
     }
-    if (!F->general_ok) return EQ_OK;
     // from a residual of about the right-hand side to the tolerance
     const double todo = std::log(1.0 / std::max(b->solver.rtol, 1e-15));
     const int n = worst > 0.0 ? (int)(todo / std::log(1.0 / worst)) + 1 : 3;
@@ -795,15 +788,31 @@ int fast_refresh(eq_batch* b)
         hipFree(F->d_stiff);
         F->d_stiff = nullptr;
         F->stiff_stride = b->levels[0].pool;
-        if (aniso && hipMalloc((void**)&F->d_stiff, sizeof(double) * 3 * F->stiff_stride) != hipSuccess)
-            return set_error(EQ_ERR_NOMEM, "stiffness weights");
+        if (aniso && hipMalloc((void**)&F->d_stiff, sizeof(double) * 3 * F->stiff_stride) != hipSuccess) {
+            F->d_stiff = nullptr;
+            hipGetLastError();
+            return EQ_OK; // no room: the multigrid solvers need none
+        }
         if (aniso) EQ_HIP(hipMemset(F->d_stiff, 0, sizeof(double) * 3 * F->stiff_stride));
     }
-    if (!F->d_cheb && hipMalloc((void**)&F->d_cheb, sizeof(double2) * tab.size()) != hipSuccess)
-        return set_error(EQ_ERR_NOMEM, "fast solver tables");
+    if (!F->d_cheb && hipMalloc((void**)&F->d_cheb, sizeof(double2) * tab.size()) != hipSuccess) {
+        F->d_cheb = nullptr;
+        hipGetLastError();
+        return EQ_OK;
+    }
     EQ_HIP(hipMemcpy(F->d_cheb, tab.data(), sizeof(double2) * tab.size(), hipMemcpyHostToDevice));
     EQ_HIP(hipMemcpy(F->d_extra, extra.data(), sizeof(int32_t) * extra.size(), hipMemcpyHostToDevice));
+    F->general_ok = true;
     return EQ_OK;
+}
+
+// A change of tensor fields or velocities that fails part of the way leaves
+// problems with coefficients that the tables here do not cover (a tensor
+// without stiffness weights): until fast_refresh has seen it through, steps
+// with varying coefficients take the multigrid solvers.
+void fast_forget(eq_batch* b)
+{
+    if (b->fast) b->fast->general_ok = false;
 }
 
 // Whether this step takes the fast solver: the cycle options are at their

@@ -332,7 +332,8 @@ void free_stage(eq_batch* b);
 // next step takes it; one solve (handled = false: the multigrid solver has to
 // go on); graphs and plans dropped
 int fast_build(eq_batch* b);
-int fast_refresh(eq_batch* b); // after a change of tensor fields or velocities
+void fast_forget(eq_batch* b); // before a change of tensor fields or velocities,
+int fast_refresh(eq_batch* b); // and after it
 bool fast_applies(const eq_batch* b);
 int fast_solve(eq_batch* b, bool profiling, bool* handled);
 void fast_drop_graphs(eq_batch* b);

@@ -4939,6 +4939,7 @@ static int set_tensor_checked(eq_batch* b, int32_t prob, const double* D11, cons
         b->tens_bounds.resize(b->nprob, {1.0, 1.0});
         b->tens_bounds[prob] = {lo, hi};
     }
+    fast_forget(b);
     return b->mixed ? set_tensor_impl<float>(b, prob, D11, D22, D12) : set_tensor_impl<double>(b, prob, D11, D22, D12);
 }
 
@@ -5188,6 +5189,7 @@ int eq_batch_set_velocity(eq_batch* b, int32_t prob, const double* vx, size_t n)
     if (vx && P.fd) return set_error(EQ_ERR_INVALID, "the finite-difference scheme has no advection");
     if (vx && P.aniso) return set_error(EQ_ERR_INVALID, "advection and a tensor field together are not supported");
     hipSetDevice(b->device);
+    fast_forget(b);
     const int rc = b->mixed ? set_velocity_impl<float>(b, prob, vx) : set_velocity_impl<double>(b, prob, vx);
     if (rc) return rc;
     return refresh_general(b);

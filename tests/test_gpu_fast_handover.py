@@ -73,3 +73,33 @@ def test_a_tensor_set_over_the_cells_tensor(eqf, oracle, solver):
             assert fb.profile_read(eqf.KERNEL_FINISH)[0] == 0 and its[step] <= max(its[:2]), its
             ref, _ = oracle.step(p, before, "lu", D11=t[0], D22=t[1], D12=t[2])
             assert _rel(fb.download(0), ref) <= 1e-9, step
+
+
+def test_a_refused_tensor_leaves_the_other_problems(eqf, oracle):
+    """A tensor that is refused (not positive definite, found out level by
+    level) beside a problem with a velocity, which the fast solver would take:
+    that problem's steps stay the oracle's, before and after the tensor is
+    taken off again."""
+    nx, ny = 64, 33
+    walls = {oracle.TOP: (oracle.DIRICHLET, 0.0, 0.0, 0.0)}
+    args = (nx, ny, nx * H, ny * H, DT, 60.0, 0.01, 0.0)
+    rng = np.random.default_rng(4)
+    u, vel, one = rng.random((nx + 1) * (ny + 1)), 10.0 * rng.random(ny + 1), np.ones((nx + 1) * (ny + 1))
+    p = oracle.problem(*args, walls=walls)
+    p.set_velocity(vel)
+    with eqf.FieldBatch([eqf.field_desc(*args, walls)] * 2,
+                        solver=eqf.solver_desc(eqf.GMG_BICGSTAB, max_iter=100)) as fb:
+        fb.set_velocity(0, vel)
+        for step in range(3):
+            if step == 1:
+                with pytest.raises(eqf.EqError) as e:
+                    fb.set_tensor(1, -one, -one, 0.0 * one)
+                assert e.value.code == 1
+            if step == 2:
+                fb.set_tensor(1)
+            fb.upload(0, u)
+            fb.upload(1, u)
+            st = fb.step(check=False)
+            assert st.nconverged == (1 if step == 1 else 2), step
+            ref, _ = oracle.step(p, u, "lu")
+            assert _rel(fb.download(0), ref) <= 1e-9, step
