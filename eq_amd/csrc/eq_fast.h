@@ -52,6 +52,8 @@ struct FastProb {
     int32_t plan, ends;
     int32_t pair0, npairs;  // this problem's slots of row-pair partials
     int64_t mode0;          // its modes' records
+    double gain;            // what an application leaves of the error at most, squared (constant coefficients)
+    double unit;            // an update's size in the right-hand side's units, squared
 };
 
 // A mode's tridiagonal inverse along y (k_fast_lines), laid out once: forming
@@ -96,7 +98,7 @@ struct FastSolver {
     FastJob* d_lines = nullptr;  // mode groups
     FastMode* d_modes = nullptr;
     void* d_tables = nullptr;
-    double* d_partial = nullptr; // 2 per row pair
+    double* d_partial = nullptr; // 3 per row pair: residual, right-hand side, last update
     bool robin_x = false; // some left or right wall is a Robin wall
     // beyond the constant operator (tensor field, advection, Robin walls
     // across x): per problem kChebMax
@@ -393,6 +395,24 @@ __device__ __forceinline__ double scale_down(const CgState& cs, int k)
     return sizeof(T) == 4 ? ldexp(1.0, -(k == 0 ? cs.fast_e0 : cs.fast_e)) : 1.0;
 }
 
+// Whether a solve is over: the residual rr within the tolerance and, with
+// constant coefficients, the error within kFastError of it.  The residual alone
+// does not tell the error: where the last application just got there the error
+// is 3e-3 to 5e-2 of the residual (smooth fields, small dt D), up to 2e-12 of a
+// field where the V-cycle CG left 2e-14 to 1e-12; and rounding (4e-12 at
+// 2000x1000) hides how far below the tolerance the error is.  But the last
+// update is the error before it, and an application leaves the part of it that
+// the residuals show, at most `gain`.  All squared: prev the residual before
+// the last application (< 0: there was none), upd that update in the
+// right-hand side's units.  (varying: a fixed number of applications follow
+// instead, fast_refresh)
+constexpr double kFastError = 2e-4;
+__device__ __forceinline__ bool within(double rr, double tol, double prev, double upd, double gain, bool varying)
+{
+    return rr <= tol &&
+           (varying || prev < 0.0 || upd * fmin(gain, rr / prev) <= kFastError * kFastError * tol);
+}
+
 // waves per SIMD the transform kernels are compiled for
 constexpr int fast_waves(size_t elem, int NT, int V) { return V > kFastValues ? 4 : elem == 4 ? 8 : 4; }
 
@@ -656,8 +676,8 @@ __global__ __launch_bounds__(NT, GEN ? 4 : fast_waves(sizeof(T), NT, V)) void k_
     });
     block_pair<NT>(acc);
     if (threadIdx.x == 0) {
-        partial[2 * (int64_t)(f.pair0 + job.at)] = acc[0];
-        partial[2 * (int64_t)(f.pair0 + job.at) + 1] = acc[1];
+        partial[3 * (int64_t)(f.pair0 + job.at)] = acc[0];
+        partial[3 * (int64_t)(f.pair0 + job.at) + 1] = acc[1];
     }
     T* __restrict__ o0 = out + P.origin + (int64_t)i0 * P.pitch;
     const bool second = i0 + 1 <= P.ny;
@@ -669,7 +689,8 @@ __global__ __launch_bounds__(NT, GEN ? 4 : fast_waves(sizeof(T), NT, V)) void k_
     });
 }
 
-// Transform back along x and x += z, two rows a block.  GEN: one application of
+// Transform back along x and x += z, two rows a block, and the update's square
+// sum.  GEN: one application of
 // the Chebyshev iteration, d <- alpha z + beta d, x += d (d in z's scale, which
 // a solve keeps).
 template <typename T, int NT, int V, bool GEN>
@@ -679,7 +700,8 @@ __global__ __launch_bounds__(NT, fast_waves(sizeof(T), NT, V)) void k_fast_backw
                                                       const FastPlan* __restrict__ plans,
                                                       const Cx<T>* __restrict__ tab, const T* __restrict__ in,
                                                       double* __restrict__ x, const CgState* __restrict__ st,
-                                                      T* __restrict__ d, const double2* __restrict__ cheb, int k)
+                                                      T* __restrict__ d, const double2* __restrict__ cheb,
+                                                      double* __restrict__ partial, int k)
 {
     extern __shared__ char lds_raw[];
     Cx<T>* s = (Cx<T>*)lds_raw;
@@ -724,6 +746,7 @@ __global__ __launch_bounds__(NT, fast_waves(sizeof(T), NT, V)) void k_fast_backw
         be = (T)w.y;
     }
     const int jlo = (P.dmask & (1 << kLeft)) ? 1 : 0, jhi = (P.dmask & (1 << kRight)) ? N - 1 : N;
+    double acc[2] = {0.0, 0.0};
     row_transform<T, NT, V>(s, pl, tab, [&](int jj, Cx<T> v) {
         const int j = ends == kEndsDN ? N - jj : jj;
         if (ends == kEndsDD)
@@ -737,9 +760,17 @@ __global__ __launch_bounds__(NT, fast_waves(sizeof(T), NT, V)) void k_fast_backw
             dr[j] = v.x;
             if (second) dr[j + pitch] = v.y;
         }
-        if (!held0 && !top0) xr[j] += up * (double)v.x;
-        if (second && !held1) xr[j + pitch] += up * (double)v.y;
+        if (!held0 && !top0) {
+            xr[j] += up * (double)v.x;
+            acc[0] += (double)v.x * (double)v.x;
+        }
+        if (second && !held1) {
+            xr[j + pitch] += up * (double)v.y;
+            acc[1] += (double)v.y * (double)v.y;
+        }
     });
+    block_pair<NT>(acc);
+    if (threadIdx.x == 0) partial[3 * (int64_t)(f.pair0 + job.at) + 2] = (acc[0] + acc[1]) * (up * up);
 }
 
 // ------------------------------------------------------------ launches

@@ -60,32 +60,28 @@ __global__ __launch_bounds__(256) void k_fast_check(const FastJob* __restrict__ 
     double acc[2] = {0.0, 0.0};
     residual_pair<256, GEN>(P, rows[job.prob], 2 * job.at, u, x, stiff, sst, false, acc, [](int, double, double) {});
     block_pair<256>(acc);
-    if (threadIdx.x == 0) partial[2 * (int64_t)(fp[job.prob].pair0 + job.at)] = acc[0];
+    if (threadIdx.x == 0) partial[3 * (int64_t)(fp[job.prob].pair0 + job.at)] = acc[0];
 }
 
 // Sums a problem's row-pair partials: the same order in every block of the
 // launch.  Result in every thread.
-__device__ __forceinline__ void sum_pairs(const double* __restrict__ partial, int npairs, double* red, double& rr,
-                                          double& bb)
+__device__ __forceinline__ void sum_pairs(const double* __restrict__ partial, int npairs, double* red, double (&sum)[3])
 {
-    double a = 0.0, b = 0.0;
-    for (int q = threadIdx.x; q < npairs; q += blockDim.x) {
-        a += partial[2 * q];
-        b += partial[2 * q + 1];
-    }
-    a = wave_add(a);
-    b = wave_add(b);
+    double v[3] = {0.0, 0.0, 0.0};
+    for (int q = threadIdx.x; q < npairs; q += blockDim.x)
+#pragma unroll
+        for (int e = 0; e < 3; ++e) v[e] += partial[3 * q + e];
     const int w = threadIdx.x >> 6, nw = (blockDim.x + 63) >> 6;
-    if ((threadIdx.x & 63) == 0) {
-        red[2 * w] = a;
-        red[2 * w + 1] = b;
+#pragma unroll
+    for (int e = 0; e < 3; ++e) {
+        v[e] = wave_add(v[e]);
+        if ((threadIdx.x & 63) == 0) red[3 * w + e] = v[e];
+        sum[e] = 0.0;
     }
     __syncthreads();
-    rr = bb = 0.0;
-    for (int q = 0; q < nw; ++q) {
-        rr += red[2 * q];
-        bb += red[2 * q + 1];
-    }
+    for (int q = 0; q < nw; ++q)
+#pragma unroll
+        for (int e = 0; e < 3; ++e) sum[e] += red[3 * q + e];
 }
 
 __device__ __forceinline__ double ipow(double a, int n)
@@ -163,7 +159,7 @@ __global__ __launch_bounds__(1024, MANY && sizeof(T) == 4 && L == 16 ? 6 : 4) vo
                              const double* __restrict__ partial, CgState* st, const int32_t* __restrict__ extra,
                              int32_t* met_at, int k)
 {
-    __shared__ double red[40];                  // 32 doubles of sums, then the flags
+    __shared__ double red[50];                  // 48 doubles of sums, then the flags
     __shared__ double tot[2][16][kFastModes];   // the waves' totals, up and down
     const int t = swizzled_block();
     if (t >= njobs) return;
@@ -184,13 +180,13 @@ __global__ __launch_bounds__(1024, MANY && sizeof(T) == 4 && L == 16 ? 6 : 4) vo
     for (int l = 0; l < L; ++l) v[l] = (on && l < nl) ? col[(int64_t)l * P.pitch] : (T)0;
     std::conditional_t<MANY, const FastMode&, const FastMode> M = modes[f.mode0 + min(q, N)];
     if (threadIdx.x == 0) {
-        ((int*)(red + 36))[0] = k > 0 ? cs.done : 0;
-        ((int*)(red + 36))[1] = k > 0 ? met_at[P.prob] : -1;
+        ((int*)(red + 48))[0] = k > 0 ? cs.done : 0;
+        ((int*)(red + 48))[1] = k > 0 ? met_at[P.prob] : -1;
     }
-    double rr, bb;
-    sum_pairs(partial + 2 * (int64_t)f.pair0, f.npairs, red, rr, bb);
-    if (((int*)(red + 36))[0]) return;
-    if (k > 0) bb = cs.bb;
+    double sum[3];
+    sum_pairs(partial + 3 * (int64_t)f.pair0, f.npairs, red, sum);
+    if (((int*)(red + 48))[0]) return;
+    const double rr = sum[0], bb = k > 0 ? cs.bb : sum[1];
     // the first launch settles the scale (fast_e0 is not written here, so every block finds the same)
     int e = 0, drop = 0;
     if (sizeof(T) == 4 && k == 0) {
@@ -204,8 +200,9 @@ __global__ __launch_bounds__(1024, MANY && sizeof(T) == 4 && L == 16 ? 6 : 4) vo
     }
     const int app = k == 0 ? 0 : max(0, k - cs.fast_void); // applications done
     // (a block that already reads the first block's entry takes the same way)
-    const bool conv = rr <= cs.tol2 * bb;
-    int first = ((int*)(red + 36))[1];
+    const bool conv = within(rr, cs.tol2 * bb, app > 0 ? cs.fast_rr[(k - 1) & 1] : -1.0, f.unit * sum[2], f.gain,
+                             extra[job.prob] > 0);
+    int first = ((int*)(red + 48))[1];
     if (conv && first < 0) first = app;
     const bool stop = conv && app >= first + extra[job.prob];
     if (job.at == 0 && threadIdx.x == 0) {
@@ -214,6 +211,7 @@ __global__ __launch_bounds__(1024, MANY && sizeof(T) == 4 && L == 16 ? 6 : 4) vo
             cs.fast_void = drop;
             cs.fast_e = e;
         }
+        cs.fast_rr[k & 1] = rr; // (the other one is being read)
         met_at[P.prob] = first;
         cs.done = stop ? 1 : 0;
         if (stop) {
@@ -294,7 +292,7 @@ __global__ __launch_bounds__(256) void k_fast_commit(const FastJob* __restrict__
                                                      const double* __restrict__ x, const double* __restrict__ partial,
                                                      CgState* st, const int32_t* __restrict__ extra, int32_t* met_at, int k)
 {
-    __shared__ double red[16];
+    __shared__ double red[12];
     __shared__ int was, met;
     const int t = swizzled_block();
     if (t >= njobs) return;
@@ -306,12 +304,14 @@ __global__ __launch_bounds__(256) void k_fast_commit(const FastJob* __restrict__
         was = cs.done;
         met = met_at[P.prob];
     }
-    double rr, bb;
-    sum_pairs(partial + 2 * (int64_t)f.pair0, f.npairs, red, rr, bb);
+    double sum[3];
+    sum_pairs(partial + 3 * (int64_t)f.pair0, f.npairs, red, sum);
     if (was == 2) return;
+    const double rr = sum[0];
     // (a block that already reads the first block's `done` takes the same way)
-    const bool conv = rr <= cs.tol2 * cs.bb;
     const int app = k - cs.fast_void;
+    const bool conv = within(rr, cs.tol2 * cs.bb, app > 0 ? cs.fast_rr[(k - 1) & 1] : -1.0, f.unit * sum[2], f.gain,
+                             extra[job.prob] > 0);
     const int first = conv && met < 0 ? app : met;
     const bool over = was || (conv && app >= first + extra[job.prob]);
     if (job.at == 0 && threadIdx.x == 0) {
@@ -629,6 +629,15 @@ static int fast_build_t(eq_batch* b, FastSolver* F)
         fp[p].npairs = (P.ny + 2) / 2;
         pairs += fp[p].npairs;
         fp[p].mode0 = modes;
+        // the mass couplings that P spreads (sin a sin b / 6 h^2 of the mass
+        // against 2 (1 - cos a) + 2 (1 - cos b) of dt D), or the transforms'
+        // rounding (measured 1.4e-6 and below 1e-13 of the residual)
+        const eq_field_desc& D = b->descs[p];
+        const double mass = P.fd ? 0.0 : (1.0 + D.dt * D.gamma) * P.hx * P.hy / (12.0 * D.dt * D.D);
+        const double gain = std::max(mass, sizeof(T) == 4 ? 5e-7 : 1e-14);
+        fp[p].gain = gain * gain;
+        const double unit = (1.0 + D.dt * D.gamma) * P.hx * P.hy;
+        fp[p].unit = unit * unit;
         modes += P.nx + 1;
         rows = std::max(rows, P.ny + 1);
         for (int ci = 0; ci < 3; ++ci)
@@ -676,7 +685,7 @@ static int fast_build_t(eq_batch* b, FastSolver* F)
         (rc = put_table(&F->d_jobs, jobs, s)) || (rc = put_table(&F->d_lines, lines, s)))
         return rc;
     if (hipMalloc(&F->d_tables, sizeof(Cx<T>) * tab) != hipSuccess ||
-        hipMalloc((void**)&F->d_partial, sizeof(double) * 2 * pairs) != hipSuccess ||
+        hipMalloc((void**)&F->d_partial, sizeof(double) * 3 * pairs) != hipSuccess ||
         hipMalloc((void**)&F->d_modes, sizeof(FastMode) * modes) != hipSuccess ||
         hipMalloc((void**)&F->d_extra, sizeof(int32_t) * b->nprob) != hipSuccess ||
         hipMalloc((void**)&F->d_met, sizeof(int32_t) * b->nprob) != hipSuccess)

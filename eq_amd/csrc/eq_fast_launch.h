@@ -47,7 +47,7 @@ void fast_backward(eq_batch* b, int k)
                    dim3(grid8(c.njobs)), dim3(NT), c.lds, b->stream, (const FastJob*)F->d_jobs + c.job0, c.njobs,
                    (const LevelProb*)b->levels[0].d_probs, (const FastProb*)F->d_probs, (const FastPlan*)F->d_plans,
                    (const Cx<T>*)F->d_tables, (const T*)b->z, b->xprev, (const CgState*)b->d_state, (T*)b->q,
-                   (const double2*)F->d_cheb, k);
+                   (const double2*)F->d_cheb, F->d_partial, k);
         });
 }
 

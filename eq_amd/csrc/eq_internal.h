@@ -69,6 +69,7 @@ struct CgState {
     // this solve that only set the scale (0 or 1); the scale's exponent at a
     // solve's start and from its second launch on
     int32_t fast_iter, fast_void, fast_e0, fast_e;
+    double fast_rr[2];      // the residuals of its last two launches, even and odd
 };
 
 struct FastSolver; // eq_fast.hip
