@@ -690,9 +690,8 @@ __global__ __launch_bounds__(NT, GEN ? 4 : fast_waves(sizeof(T), NT, V)) void k_
 }
 
 // Transform back along x and x += z, two rows a block, and the update's square
-// sum.  GEN: one application of
-// the Chebyshev iteration, d <- alpha z + beta d, x += d (d in z's scale, which
-// a solve keeps).
+// sum.  GEN: one application of the Chebyshev iteration, d <- alpha z + beta d,
+// x += d, with d in FP64 (as the directions of BiCGStab are).
 template <typename T, int NT, int V, bool GEN>
 __global__ __launch_bounds__(NT, fast_waves(sizeof(T), NT, V)) void k_fast_backward(const FastJob* __restrict__ jobs, int njobs,
                                                       const LevelProb* __restrict__ probs,
@@ -700,7 +699,7 @@ __global__ __launch_bounds__(NT, fast_waves(sizeof(T), NT, V)) void k_fast_backw
                                                       const FastPlan* __restrict__ plans,
                                                       const Cx<T>* __restrict__ tab, const T* __restrict__ in,
                                                       double* __restrict__ x, const CgState* __restrict__ st,
-                                                      T* __restrict__ d, const double2* __restrict__ cheb,
+                                                      double* __restrict__ d, const double2* __restrict__ cheb,
                                                       double* __restrict__ partial, int k)
 {
     extern __shared__ char lds_raw[];
@@ -738,12 +737,12 @@ __global__ __launch_bounds__(NT, fast_waves(sizeof(T), NT, V)) void k_fast_backw
     const int pitch = P.pitch;
     const bool held0 = i0 == 0 && (P.dmask & (1 << kBottom)), held1 = i0 + 1 == P.ny && (P.dmask & (1 << kTop));
     const bool top0 = i0 == P.ny && (P.dmask & (1 << kTop));
-    [[maybe_unused]] T* __restrict__ dr = GEN ? d + P.origin + (int64_t)i0 * P.pitch : nullptr;
-    [[maybe_unused]] T al = (T)1, be = (T)0;
+    [[maybe_unused]] double* __restrict__ dr = GEN ? d + P.origin + (int64_t)i0 * P.pitch : nullptr;
+    [[maybe_unused]] double al = 1.0, be = 0.0;
     if constexpr (GEN) {
         const double2 w = cheb[(int64_t)job.prob * kChebMax + min(app, kChebMax - 1)];
-        al = (T)w.x;
-        be = (T)w.y;
+        al = w.x * up;
+        be = w.y;
     }
     const int jlo = (P.dmask & (1 << kLeft)) ? 1 : 0, jhi = (P.dmask & (1 << kRight)) ? N - 1 : N;
     double acc[2] = {0.0, 0.0};
@@ -754,23 +753,29 @@ __global__ __launch_bounds__(NT, fast_waves(sizeof(T), NT, V)) void k_fast_backw
         else if (ends >= kEndsND)
             v = mul(v, tab[pl.quart + jj]);
         if (j < jlo || j > jhi) return;
+        double v0 = (double)v.x, v1 = (double)v.y;
         if constexpr (GEN) {
-            if (app > 0) v = Cx<T>{al * v.x + be * dr[j], al * v.y + (second ? be * dr[j + pitch] : (T)0)};
-            else v = Cx<T>{al * v.x, al * v.y};
-            dr[j] = v.x;
-            if (second) dr[j + pitch] = v.y;
+            v0 *= al;
+            v1 *= al;
+            if (app > 0) {
+                v0 += be * dr[j];
+                if (second) v1 += be * dr[j + pitch];
+            }
+            dr[j] = v0;
+            if (second) dr[j + pitch] = v1;
         }
+        const double sc = GEN ? 1.0 : up;
         if (!held0 && !top0) {
-            xr[j] += up * (double)v.x;
-            acc[0] += (double)v.x * (double)v.x;
+            xr[j] += sc * v0;
+            acc[0] += v0 * v0;
         }
         if (second && !held1) {
-            xr[j + pitch] += up * (double)v.y;
-            acc[1] += (double)v.y * (double)v.y;
+            xr[j + pitch] += sc * v1;
+            acc[1] += v1 * v1;
         }
     });
     block_pair<NT>(acc);
-    if (threadIdx.x == 0) partial[3 * (int64_t)(f.pair0 + job.at) + 2] = (acc[0] + acc[1]) * (up * up);
+    if (threadIdx.x == 0) partial[3 * (int64_t)(f.pair0 + job.at) + 2] = (acc[0] + acc[1]) * (GEN ? 1.0 : up * up);
 }
 
 // ------------------------------------------------------------ launches

@@ -773,9 +773,12 @@ int fast_refresh(eq_batch* b)
         // The residual has a floor of rounding (the iterate's own, times the
         // largest eigenvalue) that the error does not share, so a tighter
         // tolerance may be out of reach: a fixed number of applications takes
-        // the error down to the multigrid solvers' (another factor of 100,
-        // 1000 with flow, 10 for Robin walls alone; 3.5e-12 -> 5e-14 and 4.5e-11 -> 2e-13 of the field).
-        extra[p] = rate > 0.0 ? (int)std::ceil(std::log(P.vel ? 1000.0 : P.aniso ? 100.0 : 10.0) / std::log(1.0 / rate)) : 0;
+        // the error down to what the multigrid solvers leave at best: another
+        // factor of 1e5 with flow (BiCGStab overshoots: 4e-14 to 1e-11 of the
+        // field; a factor of 1000 left 2e-13), 300 with a tensor (CG: 2e-14 to
+        // 3e-13; 100 left up to 1e-13) and 1e4 for Robin walls alone, whose
+        // rate is small: two or three (one left 1e-13).
+        extra[p] = rate > 0.0 ? (int)std::ceil(std::log(P.vel ? 1e5 : P.aniso ? 3e2 : 1e4) / std::log(1.0 / rate)) : 0;
         most = std::max(most, extra[p]);
         double2* w = tab.data() + (size_t)p * kChebMax;
         double al = 1.0 / d;

@@ -43,10 +43,10 @@ void fast_backward(eq_batch* b, int k)
     for (const FastClass& c : F->classes)
         by_threads(c.threads, [&](auto t) {
             constexpr int NT = std::min(1024, decltype(t)::value), V = decltype(t)::value / NT * kFastValues;
-            launch(b, EQ_KERNEL_CG_UPDATE, c.nodes * (16.0 + (GEN ? 3 : 1) * sizeof(T)), k_fast_backward<T, NT, V, GEN>,
+            launch(b, EQ_KERNEL_CG_UPDATE, c.nodes * ((GEN ? 32.0 : 16.0) + sizeof(T)), k_fast_backward<T, NT, V, GEN>,
                    dim3(grid8(c.njobs)), dim3(NT), c.lds, b->stream, (const FastJob*)F->d_jobs + c.job0, c.njobs,
                    (const LevelProb*)b->levels[0].d_probs, (const FastProb*)F->d_probs, (const FastPlan*)F->d_plans,
-                   (const Cx<T>*)F->d_tables, (const T*)b->z, b->xprev, (const CgState*)b->d_state, (T*)b->q,
+                   (const Cx<T>*)F->d_tables, (const T*)b->z, b->xprev, (const CgState*)b->d_state, b->q,
                    (const double2*)F->d_cheb, F->d_partial, k);
         });
 }

@@ -10,8 +10,9 @@ pytestmark = pytest.mark.gpu
 DT = 0.1
 
 
-def _operator(nx, ny, w, h, D, gamma, vel=None):
-    """x -> (mass M x, operator A x) of the P1 "right"-diagonal mesh with closed walls, in extended precision.  The
+def _operator(nx, ny, w, h, D, gamma, vel=None, robin=0.0):
+    """x -> (mass M x, operator A x) of the P1 "right"-diagonal mesh with closed walls, or Robin walls (s = 0) of that
+    rate on the left and right, in extended precision.  The
     stiffness takes differences: entries rounded to 64 bits alone are worth 1e-12 of the solution at dt D = 6000 h^2."""
     hx, hy = np.longdouble(w) / nx, np.longdouble(h) / ny
     area = hx * hy / 2
@@ -33,17 +34,21 @@ def _operator(nx, ny, w, h, D, gamma, vel=None):
                     if v is not None:
                         c = c + gb[0] * area / 12 * (sum(at(v, p) for p in verts) + at(v, pa))
                     at(k, pa)[...] += c * (at(x, pb) - at(x, pa))
+        for e in (0, -1):
+            at = x[:, e]
+            k[:-1, e] += robin * hy * (at[:-1] / 3 + at[1:] / 6)
+            k[1:, e] += robin * hy * (at[1:] / 3 + at[:-1] / 6)
         return m.reshape(-1), ((1 + np.longdouble(DT) * gamma) * m + np.longdouble(DT) * k).reshape(-1)
     return both
 
 
-def _exact(o, p, a, u, vel=None):
+def _exact(o, p, a, u, vel=None, robin=0.0):
     """The step's solution with the top wall held at 0: the oracle's matrix factored, refined on extended residuals."""
     import scipy.sparse.linalg as sla
     rp, c, v = o.assemble(p)
     v, _ = o.apply_dirichlet(p, rp, c, v, o.assemble_rhs(p, u))
     lu = sla.splu(o.to_scipy(rp, c, v, u.size).tocsc())
-    both = _operator(*a[:4], a[5], a[6], vel)
+    both = _operator(*a[:4], a[5], a[6], vel, robin)
     b = both(u.astype(np.longdouble))[0]
     x = np.zeros(u.size, np.longdouble)
     for _ in range(4):
@@ -81,5 +86,52 @@ def test_uneven_traps(eqf, oracle, kind):
         for k, x in enumerate(u):
             fb.upload(k, x)
         fb.step()
-        err = [_rel(fb.download(k), _exact(oracle, oracle.problem(*a, walls=walls), a, u[k])) for k, a in enumerate(args)]
+        err = [_rel(fb.download(k), _exact(oracle, oracle.problem(*a, walls=walls, grid_walls=True), a, u[k])) for k, a in enumerate(args)]
     assert max(err) <= 1e-13, err
+
+
+@pytest.mark.parametrize("kind", ["MIXED_GMG_BICGSTAB", "GMG_BICGSTAB"])
+def test_velocities(eqf, oracle, kind):
+    """A channel's profile at s = 0.8 and 0.4 for the two species; the first
+    step, and one from a kept solution."""
+    rng = np.random.default_rng(22)
+    walls = {oracle.TOP: (oracle.DIRICHLET, 0.0, 0.0, 0.0)}
+    nx, ny = 301, 149
+    args = [(nx, ny, nx / 20, ny / 20, DT, D, 0.01, 0.0) for D in (400.0, 100.0)]
+    y = np.linspace(0, 1, ny + 1)
+    vel = 200.0 * y * (1 - y)
+    u = [_field(rng, nx, ny) for _ in args]
+    probs = [oracle.problem(*a, walls=walls, grid_walls=True) for a in args]
+    with eqf.FieldBatch([eqf.field_desc(*a, walls) for a in args], nspecies=2,
+                        solver=eqf.solver_desc(getattr(eqf, kind))) as fb:
+        for k, p in enumerate(probs):
+            fb.set_velocity(k, vel)
+            p.set_velocity(vel)
+            fb.upload(k, u[k])
+        for step in range(2):
+            fb.step()
+            for k, a in enumerate(args):
+                ref = _exact(oracle, probs[k], a, u[k], vel)
+                u[k] = fb.download(k)
+                assert _rel(u[k], ref) <= 1e-13, (step, k)
+
+
+@pytest.mark.parametrize("kind", ["MIXED_GMG_CG", "GMG_CG"])
+def test_robin_walls(eqf, oracle, kind):
+    rng = np.random.default_rng(23)
+    rate = 1.5
+    walls = {oracle.TOP: (oracle.DIRICHLET, 0.0, 0.0, 0.0), oracle.LEFT: (oracle.ROBIN, 0.0, rate, 0.0),
+             oracle.RIGHT: (oracle.ROBIN, 0.0, rate, 0.0)}
+    nx, ny = 227, 128
+    args = [(nx, ny, nx / 10, ny / 10, DT, D, 0.01, 0.0) for D in (400.0, 100.0, 250.0)]
+    u = [_field(rng, nx, ny) for _ in args]
+    with eqf.FieldBatch([eqf.field_desc(*a, walls) for a in args], nspecies=3,
+                        solver=eqf.solver_desc(getattr(eqf, kind))) as fb:
+        for k, x in enumerate(u):
+            fb.upload(k, x)
+        for step in range(2):
+            fb.step()
+            for k, a in enumerate(args):
+                ref = _exact(oracle, oracle.problem(*a, walls=walls, grid_walls=True), a, u[k], robin=rate)
+                u[k] = fb.download(k)
+                assert _rel(u[k], ref) <= 1e-13, (step, k)
