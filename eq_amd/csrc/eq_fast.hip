@@ -656,6 +656,7 @@ static int fast_build_t(eq_batch* b, FastSolver* F)
         while (kFastValues * nt < plans[it->second].M && nt < 2048) nt *= 2;
         thr[p] = nt; // 2048: 1024 threads of twice the values
     }
+    for (int p = 0; p < b->nprob; ++p) F->chirp.push_back((uint8_t)plans[fp[p].plan].chirp);
     std::vector<FastJob> jobs, lines;
     for (int nt = 64; nt <= 2048; nt *= 2) {
         FastClass c;
@@ -717,6 +718,40 @@ int fast_build(eq_batch* b)
     return rc || !b->fast->robin_x ? rc : fast_refresh(b);
 }
 
+// Whether the Chebyshev iteration of fast_refresh is faster than the Krylov
+// solver, which takes 5 to 6 iterations for a flow of any strength and 8 for
+// Robin walls: microseconds a step as measured from 404x154 to 3000x1800, 2
+// species (m: millions of nodes of the batch).  An application takes 28, and a million nodes in it 28 + m (FP32) or
+// 32 + 2 m (FP64; the vectors outgrow the caches), by chirp 60 or 80; problems
+// drop out one by one, and a kept solution saves 0.15 of the applications.
+// Measured, fast against Krylov: flow of s = 0.8 in FP64 900x450 1.48 ms for
+// 3.17, 901x449 (chirp) 2.14 for 3.12, 1237x611 (chirp) 3.8 for 3.5, 3000x1800
+// 13.2 for 10.8, 2999x1800 (chirp) 22.6 for 10.1; s = 0.25 at 3000x1800 7.1 for
+// 8.5; Robin walls at 2999x1800 (chirp) 5.5 for 4.7.  With tensor fields the CG
+// takes 11 to 35 iterations on seven-point tensor rows: the fast solver was 1.5
+// to 8 times faster on every size.
+static bool worth(const eq_batch* b, const std::vector<int>& apps)
+{
+    bool flow = false;
+    double m = 0.0;
+    for (const LevelProb& P : b->levels[0].probs) {
+        if (P.aniso) return true;
+        flow = flow || P.vel;
+        m += 1e-6 * (P.nx + 1) * (P.ny + 1);
+    }
+    const bool f32 = b->mixed;
+    double most = 0.0, work = 0.0;
+    for (int p = 0; p < b->nprob; ++p) {
+        const LevelProb& P = b->levels[0].probs[p];
+        const double n = apps[p] > 3 ? 0.85 * apps[p] : apps[p], large = std::min(m, 10.0);
+        const double each = b->fast->chirp[p] ? (f32 ? 60.0 : 80.0) : (f32 ? 28.0 + large : 32.0 + 2.0 * large);
+        most = std::max(most, n);
+        work += n * each * 1e-6 * (P.nx + 1) * (P.ny + 1);
+    }
+    const double krylov = flow ? (f32 ? 1950.0 + 570.0 * m : 2300.0 + 750.0 * m) : 880.0 + (f32 ? 225.0 : 325.0) * m;
+    return 150.0 + 28.0 * most + work <= 0.92 * krylov;
+}
+
 // Varying coefficients: the spectrum of P^-1 A, with P the constant operator
 // (tensor 1, no flow), is known beforehand.  The stiffness of a tensor field
 // lies between its eigenvalues' bounds times the isotropic one, triangle by
@@ -741,6 +776,10 @@ int fast_refresh(eq_batch* b)
     const bool bicg = b->solver.kind == EQ_SOLVER_GMG_BICGSTAB || b->solver.kind == EQ_SOLVER_MIXED_GMG_BICGSTAB;
     std::vector<double2> tab((size_t)b->nprob * kChebMax, make_double2(1.0, 0.0));
     std::vector<int32_t> extra(b->nprob, 0);
+    std::vector<int> apps(b->nprob, 3);
+    // from a residual of about the right-hand side to the tolerance
+    const double todo = std::log(1.0 / std::max(b->solver.rtol, 1e-15));
+    auto needed = [&](double rate) { return rate > 0.0 ? (int)(todo / std::log(1.0 / rate)) + 1 : 3; };
     double worst = 0.0;
     int most = 0;
     for (int p = 0; p < b->nprob; ++p) {
@@ -780,6 +819,7 @@ int fast_refresh(eq_batch* b)
         // rate is small: two or three (one left 1e-13).
         extra[p] = rate > 0.0 ? (int)std::ceil(std::log(P.vel ? 1e5 : P.aniso ? 3e2 : 1e4) / std::log(1.0 / rate)) : 0;
         most = std::max(most, extra[p]);
+        apps[p] = needed(rate) + extra[p];
         double2* w = tab.data() + (size_t)p * kChebMax;
         double al = 1.0 / d;
         w[0] = make_double2(al, 0.0);
@@ -788,10 +828,8 @@ int fast_refresh(eq_batch* b)
             w[k] = make_double2(al, d * al - 1.0);
         }
     }
-    // from a residual of about the right-hand side to the tolerance
-    const double todo = std::log(1.0 / std::max(b->solver.rtol, 1e-15));
-    const int n = worst > 0.0 ? (int)(todo / std::log(1.0 / worst)) + 1 : 3;
-    for (int& r : F->recent[1]) r = std::min(n + most, FastSolver::kGraphs - 1);
+    if ((worst > 0.0) && !worth(b, apps)) return EQ_OK;
+    for (int& r : F->recent[1]) r = std::min(needed(worst) + most, FastSolver::kGraphs - 1);
     EQ_HIP(hipStreamSynchronize(b->stream));
     bool aniso = false;
     for (const LevelProb& P : b->levels[0].probs) aniso = aniso || P.aniso;

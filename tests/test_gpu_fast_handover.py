@@ -103,3 +103,26 @@ def test_a_refused_tensor_leaves_the_other_problems(eqf, oracle):
             assert st.nconverged == (1 if step == 1 else 2), step
             ref, _ = oracle.step(p, u, "lu")
             assert _rel(fb.download(0), ref) <= 1e-9, step
+
+
+@pytest.mark.parametrize("kind,nx,ny,walls,flow,fast", [
+    ("GMG_BICGSTAB", 404, 154, "top", True, True), ("GMG_BICGSTAB", 1237, 611, "top", True, False),
+    ("MIXED_GMG_BICGSTAB", 901, 449, "top", True, True), ("MIXED_GMG_BICGSTAB", 2999, 1000, "top", True, False),
+    ("GMG_BICGSTAB", 2999, 1000, "top", False, True), ("GMG_CG", 404, 154, "sides", False, True),
+    ("GMG_CG", 2999, 1800, "sides", False, False), ("MIXED_GMG_CG", 2999, 1800, "top", False, True)])
+def test_the_faster_solver_is_taken(eqf, oracle, kind, nx, ny, walls, flow, fast):
+    """Flow and Robin walls across x go by the measured times of both solvers;
+    without either every size is the fast solver's."""
+    w = {oracle.TOP: (oracle.DIRICHLET, 0.0, 0.0, 0.0)}
+    if walls == "sides":
+        w[oracle.LEFT] = w[oracle.RIGHT] = (oracle.ROBIN, 0.0, 1.5, 0.2)
+    descs = [eqf.field_desc(nx, ny, nx * 0.1, ny * 0.1, DT, D, 0.01, 0.0, w) for D in (400.0, 100.0)]
+    y = np.linspace(0, 1, ny + 1)
+    with eqf.FieldBatch(descs, nspecies=2, solver=eqf.solver_desc(getattr(eqf, kind))) as fb:
+        fb.profile(eqf.KERNEL_FINISH)
+        for p in range(2):
+            if flow:
+                fb.set_velocity(p, 200.0 * y * (1 - y))
+            fb.upload(p, np.random.default_rng(p).random((nx + 1) * (ny + 1)))
+        assert fb.step().nconverged == 2
+        assert (fb.profile_read(eqf.KERNEL_FINISH)[0] == 0) == fast
