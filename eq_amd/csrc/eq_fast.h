@@ -108,6 +108,7 @@ struct FastSolver {
     int32_t* d_extra = nullptr;  // per problem: applications after the tolerance is met,
     int32_t* d_met = nullptr;    // and where it first was (-1: not yet)
     bool general_ok = false;
+    int rest = 0, last_rest = 0; // steps that leave the solver out after it gave up, and how many the last time
     std::vector<uint8_t> chirp; // per problem: its transforms are chirps
     // tensor fields: the stiffness weights of every node to its W, S and SW
     // neighbour (three arrays of level 0's layout, zero in the frame), formed

@@ -870,7 +870,7 @@ void fast_forget(eq_batch* b)
 // coefficients vary their bounds and the iteration limit allow it.
 bool fast_applies(const eq_batch* b)
 {
-    if (!b->fast) return false;
+    if (!b->fast || b->fast->rest > 0) return false;
     eq_solver_desc d;
     eq_solver_default(&d);
     const eq_solver_desc& S = b->solver;
@@ -987,16 +987,26 @@ static int fast_solve_t(eq_batch* b, bool profiling, bool* handled)
         for (int p = 0; p < b->nprob; ++p) all = all && b->h_state[p].done;
         if (all) break;
         if (k0 >= give_up) {
+            // what holds it back (a tolerance below rounding, say) may well
+            // hold at the next step: twice as many without it each time
+            F->last_rest = std::min(63, 2 * F->last_rest + 1);
+            F->rest = F->last_rest;
             *handled = false;
             return EQ_OK;
         }
         chunk = std::min(2, give_up - k0);
     }
+    F->last_rest = 0;
     int most = 1;
     for (int p = 0; p < b->nprob; ++p) most = std::max(most, b->h_state[p].iter);
     recent[F->at[gen]] = std::min(most, FastSolver::kGraphs - 1);
     F->at[gen] = (F->at[gen] + 1) & 3;
     return EQ_OK;
+}
+
+void fast_rest(eq_batch* b)
+{
+    if (b->fast && b->fast->rest > 0) --b->fast->rest;
 }
 
 int fast_solve(eq_batch* b, bool profiling, bool* handled)

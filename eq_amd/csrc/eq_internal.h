@@ -337,6 +337,7 @@ void fast_forget(eq_batch* b); // before a change of tensor fields or velocities
 int fast_refresh(eq_batch* b); // and after it
 bool fast_applies(const eq_batch* b);
 int fast_solve(eq_batch* b, bool profiling, bool* handled);
+void fast_rest(eq_batch* b); // a step is solved without it
 void fast_drop_graphs(eq_batch* b);
 void fast_free(eq_batch* b);
 } // namespace eqk

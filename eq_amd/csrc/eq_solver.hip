@@ -4435,7 +4435,10 @@ static int run_multigrid(eq_batch* b, eq_step_stats* stats);
 // from the same fields; the problems already solved keep their result.
 static int run_solve(eq_batch* b, eq_step_stats* stats)
 {
-    if (!fast_applies(b)) return run_multigrid(b, stats);
+    if (!fast_applies(b)) {
+        fast_rest(b);
+        return run_multigrid(b, stats);
+    }
     const auto t0 = std::chrono::steady_clock::now();
     bool profiling = false, handled = true;
     for (int k = 0; k < EQ_KERNEL_COUNT_; ++k) profiling = profiling || b->prof[k].enabled;

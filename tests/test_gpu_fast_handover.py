@@ -126,3 +126,22 @@ def test_the_faster_solver_is_taken(eqf, oracle, kind, nx, ny, walls, flow, fast
             fb.upload(p, np.random.default_rng(p).random((nx + 1) * (ny + 1)))
         assert fb.step().nconverged == 2
         assert (fb.profile_read(eqf.KERNEL_FINISH)[0] == 0) == fast
+
+
+def test_a_give_up_is_remembered(eqf, oracle):
+    """A tolerance below rounding: the fast solver tries again after 1, 3, 7, ...
+    steps of the cycles.  A try shows in the launches of the updates: 32 more."""
+    nx, ny = 70, 41
+    walls = {oracle.TOP: (oracle.DIRICHLET, 0.0, 0.0, 0.0)}
+    d = eqf.field_desc(nx, ny, nx * H, ny * H, DT, 60.0, 0.01, 0.0, walls)
+    u = np.random.default_rng(1).random((nx + 1) * (ny + 1))
+    counts = []
+    with eqf.FieldBatch([d], solver=eqf.solver_desc(eqf.GMG_CG, rtol=1e-18, max_iter=40)) as fb:
+        fb.profile(eqf.KERNEL_CG_UPDATE)
+        fb.upload(0, u)
+        for step in range(12):
+            before = fb.profile_read(eqf.KERNEL_CG_UPDATE)[0]
+            fb.step(check=False)
+            counts.append(fb.profile_read(eqf.KERNEL_CG_UPDATE)[0] - before)
+    # (step 0 tries too, and has fewer cycles)
+    assert [k for k in range(1, 12) if counts[k] >= counts[1] + 32] == [2, 6], counts
