@@ -23,6 +23,8 @@
 #include <cmath>
 #include <cstdio>
 #include <cstring>
+#include <memory>
+#include <new>
 #include <string>
 #include <type_traits>
 #include <vector>
@@ -4452,20 +4454,31 @@ static int run_solve(eq_batch* b, eq_step_stats* stats)
     for (int p = 0; p < b->nprob; ++p)
         if (!solved[p].done) b->h_state[p].have_prev = b->h_state[p].have_prev2 = 0;
     EQ_HIP(hipMemcpyAsync(b->d_state, b->h_state, sizeof(CgState) * b->nprob, hipMemcpyHostToDevice, b->stream));
+    // the problems that did get there keep their solutions, in host memory
+    // where the device has no room for them
     const size_t bytes = sizeof(double) * b->levels[0].pool;
     double* kept = nullptr;
-    if (hipMalloc((void**)&kept, bytes) != hipSuccess) return set_error(EQ_ERR_NOMEM, "solved fields");
+    std::unique_ptr<double[]> host;
     hipStream_t s = b->stream;
-    rc = hipMemcpyAsync(kept, b->u, bytes, hipMemcpyDeviceToDevice, s) == hipSuccess
-             ? EQ_OK
-             : set_error(EQ_ERR_HIP, "solved fields");
-    const int mg = rc == EQ_OK ? run_multigrid(b, stats) : rc;
-    for (int p = 0; rc == EQ_OK && p < b->nprob; ++p) {
+    if (std::any_of(solved.begin(), solved.end(), [](const CgState& c) { return c.done != 0; })) {
+        if (hipMalloc((void**)&kept, bytes) != hipSuccess) {
+            hipGetLastError();
+            kept = nullptr;
+            host.reset(new (std::nothrow) double[b->levels[0].pool]);
+            if (!host) return set_error(EQ_ERR_NOMEM, "solved fields");
+        }
+        if (hipMemcpyAsync(kept ? kept : host.get(), b->u, bytes, hipMemcpyDefault, s) != hipSuccess) {
+            hipFree(kept);
+            return set_error(EQ_ERR_HIP, "solved fields");
+        }
+    }
+    const int mg = run_multigrid(b, stats);
+    for (int p = 0; p < b->nprob; ++p) {
         if (!solved[p].done) continue;
         const LevelProb& P = b->levels[0].probs[p];
         const size_t n = sizeof(double) * (size_t)P.pitch * (P.ny + 1);
         for (double* v : {b->u, b->xprev})
-            if (hipMemcpyAsync(v + P.origin, kept + P.origin, n, hipMemcpyDeviceToDevice, s) != hipSuccess)
+            if (hipMemcpyAsync(v + P.origin, (kept ? kept : host.get()) + P.origin, n, hipMemcpyDefault, s) != hipSuccess)
                 rc = set_error(EQ_ERR_HIP, "solved fields");
         b->h_state[p] = solved[p];
     }
@@ -4473,7 +4486,16 @@ static int run_solve(eq_batch* b, eq_step_stats* stats)
     hipFree(kept);
     if (rc != EQ_OK) return rc;
     if (mg != EQ_OK && mg != EQ_ERR_NOT_CONVERGED) return mg;
-    return report_solve(b, stats, t0);
+    // the others' iterations as their solver counts them (refinement: all inner ones)
+    const std::vector<int32_t> its = b->iters;
+    rc = report_solve(b, stats, t0);
+    int32_t most = 0;
+    for (int p = 0; p < b->nprob; ++p) {
+        if (!solved[p].done) b->iters[p] = its[p];
+        most = std::max(most, b->iters[p]);
+    }
+    if (stats) stats->iterations_max = most;
+    return rc;
 }
 
 static int run_multigrid(eq_batch* b, eq_step_stats* stats)

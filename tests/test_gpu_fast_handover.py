@@ -145,3 +145,22 @@ def test_a_give_up_is_remembered(eqf, oracle):
             counts.append(fb.profile_read(eqf.KERNEL_CG_UPDATE)[0] - before)
     # (step 0 tries too, and has fewer cycles)
     assert [k for k in range(1, 12) if counts[k] >= counts[1] + 32] == [2, 6], counts
+
+
+def test_refinement_after_a_hand_over(eqf, oracle):
+    """IR_GMG_CG at a tolerance below rounding: its own refinement runs out too,
+    and reports its inner iterations, of the problem that needed them."""
+    nx, ny = 70, 41
+    walls = {oracle.TOP: (oracle.DIRICHLET, 0.0, 0.0, 0.0)}
+    args = (nx, ny, nx * H, ny * H, DT, 60.0, 0.01, 0.0)
+    u = np.random.default_rng(1).random((nx + 1) * (ny + 1))
+    with eqf.FieldBatch([eqf.field_desc(*args, walls)] * 2, nspecies=2,
+                        solver=eqf.solver_desc(eqf.IR_GMG_CG, rtol=1e-18)) as fb:
+        fb.upload(0, np.zeros_like(u))
+        fb.upload(1, u)
+        st = fb.step(check=False)
+        its = fb.problem_stats()[0]
+        assert st.nconverged == 1 and its[0] == 0 and st.iterations_max == its[1] > 20, its
+        assert not fb.download(0).any()
+        ref, _ = oracle.step(oracle.problem(*args, walls=walls), u, "lu")
+        assert _rel(fb.download(1), ref) <= 1e-9
