@@ -953,7 +953,25 @@ static int couple_impl(eq_batch* b, int32_t t0, int32_t ntr, const int64_t* cell
         EQ_HIP(hipMemcpyAsync(&total, d_total, sizeof(int64_t), hipMemcpyDeviceToHost, s));
         EQ_HIP(hipStreamSynchronize(s));
     }
-    if (total >= ((int64_t)1 << 32)) return set_error(EQ_ERR_INVALID, "too many cell/tile pairs");
+    // the affine coupling where the pairs or the overlap rows do not fit: the
+    // walk in list order needs the geometry alone
+    auto walk = [&]() -> int {
+        if (!b->cell_scratch) {
+            if ((rc = ensure_scratch(b, head))) return rc;
+            base = (char*)b->cell_scratch;
+            geo = (CellGeo*)base;
+            d_total = (int64_t*)(base + geo_bytes);
+            d_blk = (int64_t*)(base + geo_bytes + 256 + 2 * tb_bytes);
+            geometry();
+        }
+        launch(b, EQ_KERNEL_COUPLE, gb + 24.0 * ns * nc, k_couple_affine, dim3((unsigned)ntr), dim3(kAThreads), 0, s, traps,
+               (int)t0, (const int64_t*)b->d_cell_off, (const CellGeo*)geo, (double* const*)b->d_field_ptrs, ns, d_q, d_b,
+               d_sampled, d_counts, npm, (const int64_t*)nullptr, (int64_t)0);
+        EQ_HIP(hipGetLastError());
+        return EQ_OK;
+    };
+    if (total >= ((int64_t)1 << 32))
+        return d_b ? walk() : set_error(EQ_ERR_INVALID, "too many cell/tile pairs");
     if (!fixed && !sized) b->pair_cap = std::max(b->pair_cap, total + total / 2 + 4096);
     // slots the pair buffers hold (sized: the kept capacity; else the count)
     const size_t pb = align256(sizeof(uint32_t) * (size_t)total);
@@ -980,7 +998,11 @@ static int couple_impl(eq_batch* b, int32_t t0, int32_t ntr, const int64_t* cell
         if (need > fixed->cap) return too_big(need); // nothing written outside the scratch yet
     } else if (need > b->cell_scratch_bytes) {
         // grow (keeps nothing: recompute the geometry in the new buffer)
-        if ((rc = ensure_scratch(b, need))) return rc;
+        if ((rc = ensure_scratch(b, need))) {
+            if (!d_b) return rc;
+            hipGetLastError();
+            return walk();
+        }
         base = (char*)b->cell_scratch;
         geo = (CellGeo*)base;
         d_total = (int64_t*)(base + geo_bytes);

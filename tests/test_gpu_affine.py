@@ -73,3 +73,46 @@ def test_affine_coupling(eqf, oracle, kind, ns):
                 assert np.allclose(samp[at], s_ref, rtol=1e-13, atol=1e-300)
                 for s in range(ns):
                     assert np.allclose(fb.download(ns * t + s), fields[s], rtol=1e-14, atol=1e-15), (t, s)
+
+
+def test_affine_coupling_without_room_for_its_rows(eqf, oracle):
+    """A million cells on a device with 250 MiB left: the geometry fits (130 MB),
+    the overlap rows (256 MB) do not, and the walk in list order takes the call.
+    Samples within 1e-12: sums of 300 nodes in another order, 3e-14, carried on
+    by amounts that depend on them."""
+    import torch
+    rng = np.random.default_rng(9)
+    nx, ny, n = 1000, 500, 1000000
+    cells = np.column_stack([rng.uniform(0, nx / NPM, n), rng.uniform(0, ny / NPM, n), rng.uniform(0, 3, n),
+                             rng.uniform(2, 4, n), np.ones(n)])
+    a, b, u0 = rng.uniform(0.05, 0.15, (n, 1)), -0.05 * rng.uniform(0.5, 1.0, (n, 1)), rng.random((nx + 1) * (ny + 1))
+    dev = lambda v: torch.from_numpy(np.ascontiguousarray(v)).cuda()  # noqa: E731
+    cells_d, a_d, b_d = dev(cells), dev(a), dev(b)
+    samp_d = torch.zeros((n, 1), dtype=torch.float64, device="cuda")
+    cnt_d = torch.zeros(n, dtype=torch.int32, device="cuda")
+    torch.cuda.synchronize()
+    with eqf.FieldBatch([eqf.field_desc(nx, ny, nx / NPM, ny / NPM, 0.1, 200.0)], solver=eqf.solver_desc(eqf.GMG_CG)) as fb:
+        def couple(k):
+            fb.couple_affine_dev(0, np.array([0, k], np.int64), cells_d.data_ptr(), NPM, a_d.data_ptr(), b_d.data_ptr(),
+                                 samp_d.data_ptr(), cnt_d.data_ptr())
+            fb.sync()
+        couple(100)  # the kernels and the tables of a first call
+        fb.upload(0, u0)
+        room = [torch.empty(50 << 20, dtype=torch.uint8, device="cuda") for _ in range(5)]
+        filler, size = [], 1 << 36
+        while size >= 10 << 20:  # until nothing of 10 MiB is left
+            try:
+                filler.append(torch.empty(size, dtype=torch.uint8, device="cuda"))
+            except torch.OutOfMemoryError:
+                size //= 2
+        del room
+        torch.cuda.empty_cache()
+        try:
+            couple(n)
+        finally:
+            del filler
+            torch.cuda.empty_cache()
+        fields, s_ref, c_ref = oracle.couple_affine(oracle.grid(nx + 1, ny + 1, NPM, nx / NPM, ny / NPM), cells, [u0], a, b)
+        assert np.array_equal(cnt_d.cpu().numpy(), c_ref)
+        assert np.allclose(samp_d.cpu().numpy(), s_ref, rtol=1e-12)
+        assert np.allclose(fb.download(0), fields[0], rtol=1e-12)
