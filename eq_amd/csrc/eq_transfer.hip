@@ -64,10 +64,12 @@ static void launch_rows(eq_batch* b, double* flat, double* rows, int64_t k0, int
                        p, restart);
 }
 
-// Whether the batch's device reads and writes this memory in a kernel; other
-// memory (pageable, another device's) goes through the runtime's copy.
+// Whether the batch's device reads and writes this memory in a kernel, word by
+// word; other memory (pageable, another device's, off the words' alignment)
+// goes through the runtime's copy.
 static bool reachable(const eq_batch* b, const void* p)
 {
+    if ((uintptr_t)p % sizeof(double)) return false;
     hipPointerAttribute_t a;
     if (hipPointerGetAttributes(&a, p) != hipSuccess) {
         hipGetLastError();

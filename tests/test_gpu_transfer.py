@@ -47,3 +47,23 @@ def test_host_coupling_sizes(eqf, oracle):
             assert np.array_equal(counts, c_ref)
             assert np.allclose(sampled, s_ref, rtol=1e-13)
             assert np.allclose(fb.download(0), ref[0], rtol=1e-13)
+
+
+def test_device_memory_off_the_words(eqf):
+    """A device array that starts between two words, in and out."""
+    import torch
+    nx, ny = 37, 20
+    n = (nx + 1) * (ny + 1)
+    u = np.random.default_rng(4).random(n)
+    raw = torch.zeros(8 * n + 16, dtype=torch.uint8, device="cuda")
+    raw[4:4 + 8 * n] = torch.from_numpy(u).view(torch.uint8).cuda()
+    torch.cuda.synchronize()
+    with eqf.FieldBatch([eqf.field_desc(nx, ny, 3.7, 2.0, 0.1, 100.0)], solver=eqf.solver_desc(eqf.GMG_CG)) as fb:
+        fb.upload_dev(0, raw.data_ptr() + 4, n)
+        fb.sync()
+        assert np.array_equal(fb.download(0), u)
+        raw.zero_()
+        torch.cuda.synchronize()
+        fb.download_dev(0, raw.data_ptr() + 4, n)
+        fb.sync()
+        assert np.array_equal(raw[4:4 + 8 * n].cpu().view(torch.float64).numpy(), u)
