@@ -4998,12 +4998,10 @@ static int refresh_cell_tensors_t(eq_batch* b)
 }
 
 // (the fast solver reads the finest level alone: where it takes the next step,
-// the rest waits for a multigrid solve; a captured coupling carries it all)
+// the rest waits for a multigrid solve)
 int refresh_cell_tensors(eq_batch* b)
 {
-    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-    EQ_HIP(hipStreamIsCapturing(b->stream, &cap));
-    b->coarse_tensors_stale = cap == hipStreamCaptureStatusNone && fast_applies(b);
+    b->coarse_tensors_stale = fast_applies(b);
     if (b->coarse_tensors_stale) return EQ_OK;
     return b->mixed ? refresh_cell_tensors_t<float>(b) : refresh_cell_tensors_t<double>(b);
 }
