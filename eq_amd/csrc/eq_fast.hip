@@ -707,15 +707,44 @@ static int fast_build_t(eq_batch* b, FastSolver* F)
     return rg ? rg : fast_allow_lds<T, false>(F);
 }
 
+// The cycle options at their defaults: a caller that sets them asks for that
+// multigrid cycle.
+static bool default_cycle(const eq_solver_desc& S)
+{
+    eq_solver_desc d;
+    eq_solver_default(&d);
+    // (an application is a refinement step, and those are few)
+    if (S.kind == EQ_SOLVER_IR_GMG_CG && (S.ir_max_outer != d.ir_max_outer || S.ir_inner_rtol != d.ir_inner_rtol))
+        return false;
+    return S.mg_pre == d.mg_pre && S.mg_post == d.mg_post && S.mg_omega == d.mg_omega && S.mg_omega2 == d.mg_omega2 &&
+           S.mg_coarse_max_nodes == d.mg_coarse_max_nodes && S.mg_max_levels == d.mg_max_levels &&
+           S.mg_fuse_max_nodes == d.mg_fuse_max_nodes && S.mg_fuse_pre_max_nodes == d.mg_fuse_pre_max_nodes &&
+           S.mg_bottom_lds_bytes == d.mg_bottom_lds_bytes && S.mg_fuse_pre_top == d.mg_fuse_pre_top &&
+           S.tile4_min_nodes == d.tile4_min_nodes && S.tile8_min_nodes == d.tile8_min_nodes &&
+           S.extrapolate == d.extrapolate && S.mg_level_fused == d.mg_level_fused;
+}
+
+// Varying coefficients: not by refinement steps, and an iteration limit that
+// leaves room for the applications.
+static bool may_vary(const eq_solver_desc& S) { return S.kind != EQ_SOLVER_IR_GMG_CG && S.max_iter >= kChebMax; }
+
+// The plans of a batch that may take the solver (its options, grids and walls
+// allow it), or none; where the device has no room for them, none either.
 int fast_build(eq_batch* b)
 {
-    if (b->solver.kind == EQ_SOLVER_JACOBI_CG) return EQ_OK;
-    if (!fast_shape(b)) return EQ_OK;
+    if (b->solver.kind == EQ_SOLVER_JACOBI_CG || !default_cycle(b->solver) || !fast_shape(b)) return EQ_OK;
+    if (robin_x(b->descs[0]) && !may_vary(b->solver)) return EQ_OK;
     b->fast = new (std::nothrow) FastSolver();
     if (!b->fast) return set_error(EQ_ERR_NOMEM, "host allocation");
     b->fast->robin_x = robin_x(b->descs[0]); // (all of them)
     const int rc = b->mixed ? fast_build_t<float>(b, b->fast) : fast_build_t<double>(b, b->fast);
-    return rc || !b->fast->robin_x ? rc : fast_refresh(b);
+    if (rc == EQ_ERR_NOMEM) {
+        hipStreamSynchronize(b->stream);
+        hipGetLastError();
+        fast_free(b);
+        return EQ_OK;
+    }
+    return rc || !(b->fast->robin_x || b->any_tensor) ? rc : fast_refresh(b);
 }
 
 // Whether the Chebyshev iteration of fast_refresh is faster than the Krylov
@@ -866,26 +895,13 @@ void fast_forget(eq_batch* b)
 }
 
 // Whether this step takes the fast solver: the cycle options are at their
-// defaults (a caller that sets them asks for that multigrid cycle), and where
-// coefficients vary their bounds and the iteration limit allow it.
+// defaults (autotune may have changed them since the batch was created), and
+// where coefficients vary their bounds and the iteration limit allow it.
 bool fast_applies(const eq_batch* b)
 {
     if (!b->fast || b->fast->rest > 0) return false;
-    eq_solver_desc d;
-    eq_solver_default(&d);
-    const eq_solver_desc& S = b->solver;
     const bool varying = b->any_tensor || b->fast->robin_x;
-    if (varying && (!b->fast->general_ok || S.max_iter < kChebMax)) return false;
-    // (an application is a refinement step, and those are few)
-    if (S.kind == EQ_SOLVER_IR_GMG_CG &&
-        (varying || S.ir_max_outer != d.ir_max_outer || S.ir_inner_rtol != d.ir_inner_rtol))
-        return false;
-    return S.mg_pre == d.mg_pre && S.mg_post == d.mg_post && S.mg_omega == d.mg_omega && S.mg_omega2 == d.mg_omega2 &&
-           S.mg_coarse_max_nodes == d.mg_coarse_max_nodes && S.mg_max_levels == d.mg_max_levels &&
-           S.mg_fuse_max_nodes == d.mg_fuse_max_nodes && S.mg_fuse_pre_max_nodes == d.mg_fuse_pre_max_nodes &&
-           S.mg_bottom_lds_bytes == d.mg_bottom_lds_bytes && S.mg_fuse_pre_top == d.mg_fuse_pre_top &&
-           S.tile4_min_nodes == d.tile4_min_nodes && S.tile8_min_nodes == d.tile8_min_nodes &&
-           S.extrapolate == d.extrapolate && S.mg_level_fused == d.mg_level_fused;
+    return default_cycle(b->solver) && (!varying || (b->fast->general_ok && may_vary(b->solver)));
 }
 
 // ------------------------------------------------------------ host: one solve

@@ -4425,7 +4425,6 @@ static int solve_ir(eq_batch* b, eq_step_stats* stats)
     return EQ_OK;
 }
 
-// precision of the multigrid x whether any problem carries a tensor field
 namespace eqk {
 template <typename T>
 static int refresh_cell_tensors_t(eq_batch* b);
@@ -4498,6 +4497,7 @@ static int run_solve(eq_batch* b, eq_step_stats* stats)
     return rc;
 }
 
+// precision of the multigrid x whether any problem carries a tensor field
 static int run_multigrid(eq_batch* b, eq_step_stats* stats)
 {
     if (b->coarse_tensors_stale) {
@@ -5283,6 +5283,7 @@ int eq_batch_autotune(eq_batch* b, int32_t repeats, eq_solver_desc* chosen)
         b->solver.mg_post = kTuneShapes[shape][1];
         b->solver.mg_fuse_max_nodes = fuse;
         b->solver.mg_fuse_pre_top = top;
+        if (!b->fast && (rc = fast_build(b)) != EQ_OK) break; // (a batch created with another cycle)
         drop_graphs(b);
         double t = 0.0;
         bool ok = true;
