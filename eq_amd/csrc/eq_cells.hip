@@ -651,58 +651,77 @@ __global__ __launch_bounds__(kAThreads) void k_couple_affine(const TrapGrid* __r
 // (every earlier cell's window is tested, 64 at a time; covered nodes are
 // counted where the windows meet), k_affine_solve solves them, a workgroup a
 // trap.  The walk of k_couple_affine takes 4.5 us a cell whatever its size
-// (two scans of the window and three barriers of 16 wavefronts); 1000 rods on
-// 1000x500 nodes, 2 species, coupling and step: 4.76 -> 0.44 ms.  A cell with
-// more than kOverlaps earlier neighbours sends the call to k_couple_affine
+// (two scans of the window and three barriers of 16 wavefronts); the coupling
+// alone, 2 species, 1000 rods on 1000x500 nodes: 4.67 -> 0.29 ms, 10000 on
+// 2000x1000 30 -> 0.68, 100000 on 8000x4000 353 -> 29 (testing the windows is
+// quadratic in a trap's cells: the walk would draw level at millions).  A cell
+// with more than kOverlaps earlier neighbours sends the call to k_couple_affine
 // (*total above cap); random rods of 2-4 um at one per square micron have six.
+// So does one whose window meets more than kWindows earlier ones, found before
+// any node is counted, and every other cell then stops: such a call pays little
+// more than the walk (400 rods on 8x4 um: the walk alone 1.11 ms, with their
+// overlaps counted first 1.72, now 1.12).
 constexpr int kOverlaps = 32;
+constexpr int kWindows = 96;
 __global__ __launch_bounds__(256) void k_overlaps(const CellGeo* __restrict__ geo, int64_t nc,
                                                   const int64_t* __restrict__ off, int t0, double npm,
                                                   uint2* __restrict__ ov, int32_t* __restrict__ nov, int64_t* total,
                                                   int64_t cap)
 {
-    const int lane = threadIdx.x & 63;
-    const int64_t c = (int64_t)blockIdx.x * 4 + __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    __shared__ uint32_t met[4][kWindows]; // a wave's cells whose windows meet its own, in list order
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    const int64_t c = (int64_t)blockIdx.x * 4 + wave;
     if (c >= nc) return;
     const CellGeo& g = geo[c];
     const int64_t c0 = off[g.trap - t0];
-    int n = 0;
-    for (int64_t d0 = c0; d0 < c && n <= kOverlaps; d0 += 64) {
+    auto over = [&]() { return __hip_atomic_load(total, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) > cap; };
+    auto give_up = [&]() {
+        if (lane == 0) __hip_atomic_store(total, cap + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    };
+    int nw = 0;
+    for (int64_t d0 = c0; d0 < c; d0 += 64) {
         bool hit = false;
         if (d0 + lane < c) {
             const CellGeo& h = geo[d0 + lane];
             hit = h.i1 <= g.i2 && h.i2 >= g.i1 && h.j1 <= g.j2 && h.j2 >= g.j1;
         }
-        for (unsigned long long hits = __ballot(hit); hits; hits &= hits - 1) {
-            const int64_t d = d0 + __builtin_ctzll(hits);
-            const CellGeo& h = geo[d];
-            const double gx = inv_tx(g.cx, g.cy, g.cs, g.sn), gy = inv_ty(g.cx, g.cy, g.cs, g.sn);
-            const double hx = inv_tx(h.cx, h.cy, h.cs, h.sn), hy = inv_ty(h.cx, h.cy, h.cs, h.sn);
-            const int i1 = max(g.i1, h.i1), i2 = min(g.i2, h.i2), j1 = max(g.j1, h.j1), j2 = min(g.j2, h.j2);
-            int cnt = 0;
-            for (int jb = j1; jb <= j2; jb += 64) {
-                const int j = jb + lane;
-                const double X = (double)j / npm;
-                for (int ib = i1; ib <= i2; ib += 64) {
-                    const double Yl = (double)(ib + lane) / npm;
-                    const int nr = min(64, i2 - ib + 1);
-                    for (int k = 0; k < nr; ++k) {
-                        const double Y = readlane_d(Yl, k);
-                        const bool in = j <= j2 &&
-                                        (g.cnt == 0 || inside_box(g.cs * X, (-g.sn) * X, g.sn * Y, g.cs * Y, gx, gy, g.o, g.rad)) &&
-                                        (h.cnt == 0 || inside_box(h.cs * X, (-h.sn) * X, h.sn * Y, h.cs * Y, hx, hy, h.o, h.rad));
-                        cnt += __popcll(__ballot(in));
-                    }
+        const unsigned long long hits = __ballot(hit);
+        const int at = nw + __popcll(hits & ((1ull << lane) - 1));
+        if (hit && at < kWindows) met[wave][at] = (uint32_t)(d0 + lane);
+        nw += __popcll(hits);
+        if (nw > kWindows) return give_up();
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    int n = 0;
+    for (int e = 0; e < nw && n <= kOverlaps; ++e) {
+        if ((e & 7) == 0 && over()) return;
+        const int64_t d = (uint32_t)__builtin_amdgcn_readfirstlane((int)met[wave][e]);
+        const CellGeo& h = geo[d];
+        const double gx = inv_tx(g.cx, g.cy, g.cs, g.sn), gy = inv_ty(g.cx, g.cy, g.cs, g.sn);
+        const double hx = inv_tx(h.cx, h.cy, h.cs, h.sn), hy = inv_ty(h.cx, h.cy, h.cs, h.sn);
+        const int i1 = max(g.i1, h.i1), i2 = min(g.i2, h.i2), j1 = max(g.j1, h.j1), j2 = min(g.j2, h.j2);
+        int cnt = 0;
+        for (int jb = j1; jb <= j2; jb += 64) {
+            const int j = jb + lane;
+            const double X = (double)j / npm;
+            for (int ib = i1; ib <= i2; ib += 64) {
+                const double Yl = (double)(ib + lane) / npm;
+                const int nr = min(64, i2 - ib + 1);
+                for (int k = 0; k < nr; ++k) {
+                    const double Y = readlane_d(Yl, k);
+                    const bool in = j <= j2 &&
+                                    (g.cnt == 0 || inside_box(g.cs * X, (-g.sn) * X, g.sn * Y, g.cs * Y, gx, gy, g.o, g.rad)) &&
+                                    (h.cnt == 0 || inside_box(h.cs * X, (-h.sn) * X, h.sn * Y, h.cs * Y, hx, hy, h.o, h.rad));
+                    cnt += __popcll(__ballot(in));
                 }
             }
-            if (cnt == 0) continue;
-            if (lane == 0 && n < kOverlaps) ov[(int64_t)n * nc + c] = make_uint2((uint32_t)d, (uint32_t)cnt);
-            ++n;
         }
+        if (cnt == 0) continue;
+        if (lane == 0 && n < kOverlaps) ov[(int64_t)n * nc + c] = make_uint2((uint32_t)d, (uint32_t)cnt);
+        ++n;
     }
-    if (lane != 0) return;
-    nov[c] = min(n, kOverlaps);
-    if (n > kOverlaps) *total = cap + 1;
+    if (n > kOverlaps) return give_up();
+    if (lane == 0) nov[c] = n;
 }
 
 // The triangular solve, kAThreads cells at a time in list order, a thread a
@@ -1075,10 +1094,10 @@ static int couple_impl(eq_batch* b, int32_t t0, int32_t ntr, const int64_t* cell
         double* amount = (double*)((char*)e0 + amount_bytes);
         uint2* ov = (uint2*)((char*)amount + amount_bytes);
         int32_t* nov = (int32_t*)((char*)ov + ov_bytes);
-        tiles(nullptr, EQ_COUPLE_SAMPLE);
-        samples(e0);
         launch(b, kid, gb, k_overlaps, dim3((unsigned)((nc + 3) / 4)), dim3(256), 0, s, (const CellGeo*)geo, (int64_t)nc,
                (const int64_t*)b->d_cell_off, (int)t0, npm, ov, nov, d_total, (int64_t)total);
+        tiles(nullptr, EQ_COUPLE_SAMPLE);
+        samples(e0);
         launch(b, kid, 32.0 * ns * nc, k_affine_solve, dim3((unsigned)ntr), dim3(kAThreads), 0, s, (const CellGeo*)geo,
                (int64_t)nc, (const int64_t*)b->d_cell_off, ns, (const uint2*)ov, (const int32_t*)nov, (const double*)e0,
                d_q, d_b, d_sampled, amount, gate, (int64_t)total);

@@ -5,6 +5,8 @@ centre-node cells on one node, traps without cells, species counts at the edges
 of a pass.  The oracle's sequential loop is the reference: counts exact;
 samples within 1e-13 relative (sums of at most 600 nodes, 6.6e-14) and fields
 within 1e-14 (each node a handful of additions), as the existing affine test."""
+import sys
+
 import numpy as np
 import pytest
 
@@ -73,6 +75,20 @@ def test_affine_coupling(eqf, oracle, kind, ns):
                 assert np.allclose(samp[at], s_ref, rtol=1e-13, atol=1e-300)
                 for s in range(ns):
                     assert np.allclose(fb.download(ns * t + s), fields[s], rtol=1e-14, atol=1e-15), (t, s)
+
+
+@pytest.mark.parametrize("near", [80, 96, 97, 130])
+def test_affine_coupling_windows_without_overlaps(eqf, oracle, monkeypatch, near):
+    """A long rod whose window meets those of `near` small cells beside it, none
+    of which it covers: on both sides of the windows a cell may meet (96)."""
+    x, y = np.meshgrid(np.arange(2.2, 9.8, 0.3), np.arange(0.9, 5.1, 0.3))
+    away = np.abs(0.447 * (x - 6.0) - 0.894 * (y - 3.0)) > 0.9
+    c = np.zeros((near + 1, 5))
+    c[:near, 0], c[:near, 1] = x[away][:near] + 0.01, y[away][:near] + 0.01
+    c[:near, 3], c[:near, 4] = 0.15, 0.1
+    c[near] = 6.0, 3.0, 0.4636, 10.0, 1.0
+    monkeypatch.setattr(sys.modules[__name__], "_cells", lambda kind, rng: [(120, 60, c), (120, 60, c[:3])])
+    test_affine_coupling(eqf, oracle, "windows", 2)
 
 
 def test_affine_coupling_without_room_for_its_rows(eqf, oracle):
