@@ -5,9 +5,7 @@
 #pragma once
 
 #include <algorithm>
-#include <chrono>
 #include <cmath>
-#include <cstdio>
 #include <cstring>
 #include <map>
 #include <new>
@@ -408,7 +406,7 @@ __device__ __forceinline__ double scale_down(const CgState& cs, int k)
 // the last application (< 0: there was none), upd that update in the
 // right-hand side's units.  (varying: a fixed number of applications follow
 // instead, fast_refresh)
-constexpr double kFastError = 2e-4;
+constexpr double kFastError = 1e-4;
 __device__ __forceinline__ bool within(double rr, double tol, double prev, double upd, double gain, bool varying)
 {
     return rr <= tol &&

@@ -631,10 +631,10 @@ static int fast_build_t(eq_batch* b, FastSolver* F)
         fp[p].mode0 = modes;
         // the mass couplings that P spreads (sin a sin b / 6 h^2 of the mass
         // against 2 (1 - cos a) + 2 (1 - cos b) of dt D), or the transforms'
-        // rounding (measured 1.4e-6 and below 1e-13 of the residual)
+        // rounding (FP64: 1e-15 to 4e-15 of the field)
         const eq_field_desc& D = b->descs[p];
         const double mass = P.fd ? 0.0 : (1.0 + D.dt * D.gamma) * P.hx * P.hy / (12.0 * D.dt * D.D);
-        const double gain = std::max(mass, sizeof(T) == 4 ? 5e-7 : 1e-14);
+        const double gain = std::max(mass, sizeof(T) == 4 ? 5e-7 : 3e-15);
         fp[p].gain = gain * gain;
         const double unit = (1.0 + D.dt * D.gamma) * P.hx * P.hy;
         fp[p].unit = unit * unit;
