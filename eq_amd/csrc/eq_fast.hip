@@ -13,13 +13,15 @@
 // the step meets: two to four applications from the last step's solution,
 // where the V-cycle needed nine to ten iterations of five times the cost).
 // The residual b - A x is formed in FP64 from u and x themselves every time,
-// so the stop test is on the true residual and nothing is carried along.
+// so the stop test is on the true residual, and on the error that the last
+// update shows (within).
 // The finite-difference scheme is separable exactly.
 //
 // Measured per time step, couple + solve + fields out, against the V-cycle
-// CG: 2000x1000, 2 species 2.57 -> 0.39 ms (FP64 3.04 -> 0.44), 1237x611 (a
-// chirp length) 2.01 -> 0.33, 12 uneven traps 3.32 -> 1.03, 512 uneven traps
-// 69.8 -> 28.2; errors against a 64-bit solve 4e-15 to 6e-13.
+// CG: 2000x1000, 2 species 2.57 -> 0.40 ms (FP64 3.04 -> 0.50), 1237x611 (a
+// chirp length) 2.00 -> 0.41, 12 uneven traps 3.31 -> 1.12, 512 uneven traps
+// 69.6 -> 31.6; errors against a 64-bit solve 1e-15 to 2e-14, where the CG
+// left 2e-14 to 1e-12.
 //
 // What bounds the transforms: vector issue and latency, not bandwidth
 // (2000x1000: forward 34 us, backward 28, where the bytes take 18 and 14).
@@ -525,11 +527,12 @@ static double robin_part(const eq_field_desc& d)
 
 // Whether the batch's grids and walls allow the solver: x walls closed or
 // held (their transforms diagonalise the x matrices) or Robin walls of at most
-// twice the closed operator (over 20 applications there; in every problem of
-// the batch or none: mixed batches keep the multigrid solvers, whose iteration
-// counts on them are relied on), rows that fit a block,
-// and dt D of at least the square of the larger spacing, where the
-// separable matrix is within a tenth of the operator.
+// twice the closed operator (over 20 applications there), rows that fit a
+// block, and dt D of at least the square of the larger spacing, where the
+// separable matrix is within a tenth of the operator.  Robin walls across x in
+// some problems only would go the same way (the weights are per problem); such
+// batches are left to the multigrid solvers, whose fused and separate levels
+// are compared with one another on one, by their iteration counts.
 static bool fast_shape(const eq_batch* b)
 {
     const size_t elem = b->mixed ? sizeof(Cx<float>) : sizeof(Cx<double>);
@@ -791,10 +794,10 @@ static bool worth(const eq_batch* b, const std::vector<int>& apps)
 // ellipse (Manteuffel, Numer. Math. 28, 1977) converges at a known rate, with
 // no inner products: three launches an application, as without them.
 // Per step against the V-cycle CG and BiCGStab: a cell tensor of contrast 2 on
-// 800x400 4.50 -> 0.99 ms (18 applications of 45 us), a flow of s = 0.8 on
-// 901x449 2.54 -> 1.6 (26 of 56 us).
-// Robin walls at a rate of 1.5 on the left and right, 1057x810 in FP64: 2.74 ->
-// 1.41 (six applications).
+// 800x400 4.46 -> 1.07 ms (19 applications), a flow of s = 0.8 on 901x449 2.54
+// -> 2.02 (32).
+// Robin walls at a rate of 1.5 on the left and right, 900x450 in FP64: 1.20 ->
+// 0.47 (nine applications).
 // Beyond a rate of 1/2 an application the multigrid solvers are taken (a
 // contrast of 9, s = 4/3): there are over 35 applications to a solve.
 int fast_refresh(eq_batch* b)

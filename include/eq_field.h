@@ -105,11 +105,16 @@ typedef enum {
 /* With the cycle options (mg_*, tile*, extrapolate, ir_*) at their defaults the
  * multigrid kinds are solved by a fast direct solver in the kind's precision
  * (same tolerance on the same FP64 residual), iterations counting its
- * applications: constant coefficients directly, tensor fields of a contrast up
- * to 9, velocities up to (8/3) sqrt(D / dt) (BiCGStab kinds) and Robin walls on
- * the left and right of every problem by a Chebyshev iteration on it (not
- * IR_GMG_CG; max_iter at least 64).  Other batches, and a caller that sets a
- * cycle, get that multigrid cycle. */
+ * applications: constant coefficients directly, tensor fields (eigenvalues
+ * within a factor of 9 of one another and of 1), velocities up to (8/3)
+ * sqrt(D / dt) (BiCGStab kinds) and Robin walls on the left and right of every
+ * problem by a Chebyshev iteration on it (not IR_GMG_CG; max_iter at least 64;
+ * velocities and Robin walls where that is the faster way).  Other batches, and
+ * a caller that sets a cycle, get that multigrid cycle.  A step that the fast
+ * solver does not bring to rtol goes on with the multigrid cycle from the
+ * step's fields, and some steps after it start there.  streams and check_every
+ * have no effect on the fast solver, and IR_GMG_CG's FP32 cycles run only where
+ * it does not. */
 
 typedef struct {
     int32_t kind;                /* eq_solver_kind                                  */
@@ -271,7 +276,9 @@ int eq_batch_set_tensor(eq_batch* b, int32_t prob, const double* D11, const doub
  *   D12 = (Dx - Dy) sin a cos a          (a = the cell's angle)
  * so the last cell covering a node wins.  The coupling call then carries the
  * tensor to the coarse levels (nearest fine node) and rebuilds the coarsest
- * inverses, all on the batch stream with no host round trip.  Dx, Dy are
+ * inverses, all on the batch stream with no host round trip (where the fast
+ * solver, which reads the finest level alone, takes the next step, that waits
+ * for a multigrid solve).  Dx, Dy are
  * AnisotropicDiffusion_Axial / _Transverse (src/main.cpp:569-570).  enable = 0:
  * constant coefficients again.  Set-up call (synchronises); P1 scheme only, not
  * with a velocity. */
