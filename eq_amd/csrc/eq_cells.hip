@@ -652,8 +652,8 @@ __global__ __launch_bounds__(kAThreads) void k_couple_affine(const TrapGrid* __r
 // counted where the windows meet), k_affine_solve solves them, a workgroup a
 // trap.  The walk of k_couple_affine takes 4.5 us a cell whatever its size
 // (two scans of the window and three barriers of 16 wavefronts); the coupling
-// alone, 2 species, 1000 rods on 1000x500 nodes: 4.67 -> 0.29 ms, 10000 on
-// 2000x1000 30 -> 0.68, 100000 on 8000x4000 353 -> 29 (testing the windows is
+// alone, 2 species, 1000 rods on 1000x500 nodes: 4.67 -> 0.28 ms, 10000 on
+// 2000x1000 30 -> 0.63, 100000 on 8000x4000 353 -> 23 (testing the windows is
 // quadratic in a trap's cells: the walk would draw level at millions).  A cell
 // with more than kOverlaps earlier neighbours sends the call to k_couple_affine
 // (*total above cap); random rods of 2-4 um at one per square micron have six.
@@ -679,16 +679,23 @@ __global__ __launch_bounds__(256) void k_overlaps(const CellGeo* __restrict__ ge
         if (lane == 0) __hip_atomic_store(total, cap + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     };
     int nw = 0;
-    for (int64_t d0 = c0; d0 < c; d0 += 64) {
-        bool hit = false;
-        if (d0 + lane < c) {
-            const CellGeo& h = geo[d0 + lane];
-            hit = h.i1 <= g.i2 && h.i2 >= g.i1 && h.j1 <= g.j2 && h.j2 >= g.j1;
+    constexpr int kAhead = 4; // windows a lane loads before it tests them
+    for (int64_t d0 = c0; d0 < c; d0 += 64 * kAhead) {
+        int4 box[kAhead];
+#pragma unroll
+        for (int q = 0; q < kAhead; ++q) {
+            const CellGeo& h = geo[min(d0 + 64 * q + lane, c)]; // (c itself: in range, not counted)
+            box[q] = make_int4(h.i1, h.i2, h.j1, h.j2);
         }
-        const unsigned long long hits = __ballot(hit);
-        const int at = nw + __popcll(hits & ((1ull << lane) - 1));
-        if (hit && at < kWindows) met[wave][at] = (uint32_t)(d0 + lane);
-        nw += __popcll(hits);
+#pragma unroll
+        for (int q = 0; q < kAhead; ++q) {
+            const int64_t d = d0 + 64 * q + lane;
+            const bool hit = d < c && box[q].x <= g.i2 && box[q].y >= g.i1 && box[q].z <= g.j2 && box[q].w >= g.j1;
+            const unsigned long long hits = __ballot(hit);
+            const int at = nw + __popcll(hits & ((1ull << lane) - 1));
+            if (hit && at < kWindows) met[wave][at] = (uint32_t)d;
+            nw += __popcll(hits);
+        }
         if (nw > kWindows) return give_up();
     }
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
