@@ -409,9 +409,12 @@ __device__ __forceinline__ T scaled(double v, int e)
 // right-hand side's units.  (varying: a fixed number of applications follow
 // instead, fast_refresh)
 constexpr double kFastError = 1e-4;
-__device__ __forceinline__ bool within(double rr, double tol, double prev, double upd, double gain, bool varying)
+// A right-hand side without a finite norm makes every residual pass: only a
+// kept solution is one then, as for the V-cycle solvers, which take the others.
+__device__ __forceinline__ bool within(double rr, double tol, double prev, double upd, double gain, bool varying,
+                                       bool kept)
 {
-    return rr <= tol &&
+    return rr <= tol && (rr < HUGE_VAL || kept) &&
            (varying || prev < 0.0 || upd * fmin(gain, rr / prev) <= kFastError * kFastError * tol);
 }
 

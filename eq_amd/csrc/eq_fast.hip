@@ -203,7 +203,7 @@ __global__ __launch_bounds__(1024, MANY && sizeof(T) == 4 && L == 16 ? 6 : 4) vo
     const int app = k == 0 ? 0 : max(0, k - cs.fast_void); // applications done
     // (a block that already reads the first block's entry takes the same way)
     const bool conv = within(rr, cs.tol2 * bb, app > 0 ? cs.fast_rr[(k - 1) & 1] : -1.0, f.unit * sum[2], f.gain,
-                             extra[job.prob] > 0);
+                             extra[job.prob] > 0, cs.have_prev != 0);
     int first = ((int*)(red + 48))[1];
     if (conv && first < 0) first = app;
     const bool stop = conv && app >= first + extra[job.prob];
@@ -295,7 +295,7 @@ __global__ __launch_bounds__(256) void k_fast_commit(const FastJob* __restrict__
                                                      CgState* st, const int32_t* __restrict__ extra, int32_t* met_at, int k)
 {
     __shared__ double red[12];
-    __shared__ int was, met;
+    __shared__ int was, met, have;
     const int t = swizzled_block();
     if (t >= njobs) return;
     const FastJob job = jobs[t];
@@ -305,15 +305,17 @@ __global__ __launch_bounds__(256) void k_fast_commit(const FastJob* __restrict__
     if (threadIdx.x == 0) {
         was = cs.done;
         met = met_at[P.prob];
+        have = cs.have_prev;
     }
     double sum[3];
     sum_pairs(partial + 3 * (int64_t)f.pair0, f.npairs, red, sum);
     if (was == 2) return;
     const double rr = sum[0];
+    const bool kept = have != 0;
     // (a block that already reads the first block's `done` takes the same way)
     const int app = k - cs.fast_void;
     const bool conv = within(rr, cs.tol2 * cs.bb, app > 0 ? cs.fast_rr[(k - 1) & 1] : -1.0, f.unit * sum[2], f.gain,
-                             extra[job.prob] > 0);
+                             extra[job.prob] > 0, kept);
     const int first = conv && met < 0 ? app : met;
     const bool over = was || (conv && app >= first + extra[job.prob]);
     if (job.at == 0 && threadIdx.x == 0) {

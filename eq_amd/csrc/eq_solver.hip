@@ -4449,9 +4449,13 @@ static int run_solve(eq_batch* b, eq_step_stats* stats)
     if (handled) return report_solve(b, stats, t0);
     const std::vector<CgState> solved(b->h_state, b->h_state + b->nprob);
     // the iterates that did not get there are no start (they may have stalled
-    // or diverged): those problems start from their fields
-    for (int p = 0; p < b->nprob; ++p)
-        if (!solved[p].done) b->h_state[p].have_prev = b->h_state[p].have_prev2 = 0;
+    // or diverged), nor are their residuals a result: those problems start
+    // from their fields
+    for (int p = 0; p < b->nprob; ++p) {
+        if (solved[p].done) continue;
+        b->h_state[p].have_prev = b->h_state[p].have_prev2 = 0;
+        b->h_state[p].rr_true = 0.0;
+    }
     EQ_HIP(hipMemcpyAsync(b->d_state, b->h_state, sizeof(CgState) * b->nprob, hipMemcpyHostToDevice, b->stream));
     // the problems that did get there keep their solutions, in host memory
     // where the device has no room for them

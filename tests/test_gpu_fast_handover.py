@@ -164,3 +164,29 @@ def test_refinement_after_a_hand_over(eqf, oracle):
         assert not fb.download(0).any()
         ref, _ = oracle.step(oracle.problem(*args, walls=walls), u, "lu")
         assert _rel(fb.download(1), ref) <= 1e-9
+
+
+@pytest.mark.parametrize("kind", ["GMG_CG", "MIXED_GMG_CG", "IR_GMG_CG"])
+@pytest.mark.parametrize("spoil", ["infinity", "nan", "large"])
+def test_fields_without_a_finite_norm(eqf, oracle, kind, spoil):
+    """An infinity or a NaN in a fresh field, and values whose squares overflow,
+    end as they do with the cycles: the same error, or the same field."""
+    nx, ny = 70, 41
+    walls = {oracle.TOP: (oracle.DIRICHLET, 0.0, 0.0, 0.0)}
+    d = eqf.field_desc(nx, ny, nx * H, ny * H, DT, 60.0, 0.01, 0.0, walls)
+    u = np.random.default_rng(6).random((nx + 1) * (ny + 1))
+    u[-(nx + 1):] = 0.0
+    if spoil == "large":
+        u = np.ldexp(u, 600)
+    else:
+        u[500] = {"infinity": np.inf, "nan": np.nan}[spoil]
+    ends = []
+    for options in ({}, {"mg_coarse_max_nodes": 255}):
+        with eqf.FieldBatch([d], solver=eqf.solver_desc(getattr(eqf, kind), max_iter=70, **options)) as fb:
+            fb.upload(0, u)
+            try:
+                fb.step()
+                ends.append(fb.download(0))
+            except eqf.EqError as e:
+                ends.append(np.array([float(e.code)]))
+    assert np.array_equal(*ends), [e[:3] for e in ends]
